@@ -84,7 +84,7 @@ def timed_segments(k):
 
 def traffic_from_profiles(name, kernel="k_step"):
     """HBM bytes per launch of the kernel measured by rocprofv3 --pmc, if recorded."""
-    path = os.path.join(ROOT, "profiles", f"traffic_{name}{'_step2' if kernel == 'k_step2' else ''}.json")
+    path = os.path.join(ROOT, "profiles", f"traffic_{name}{'_sweep' if kernel == 'k_sweep' else ''}.json")
     if not os.path.exists(path):
         return None
     with open(path) as f:
@@ -96,7 +96,7 @@ def valu_per_node_from_profiles(name, kernel="k_step"):
     """VALU instructions of one launch of the kernel per 64 nodes of the
     lattice (SQ_INSTS_VALU x 64 / nodes) measured by rocprofv3 --pmc, if
     recorded."""
-    path = os.path.join(ROOT, "profiles", f"instructions_{name}{'_step2' if kernel == 'k_step2' else ''}.json")
+    path = os.path.join(ROOT, "profiles", f"instructions_{name}{'_sweep' if kernel == 'k_sweep' else ''}.json")
     if not os.path.exists(path):
         return None
     with open(path) as f:
@@ -545,8 +545,11 @@ def main():
     n = w["nx"] * w["ny"] * w["nz"]
     mlups = n * args.steps / wall / 1e6
     bpu = BYTES_PER_UPDATE[w["storage"]]
-    if h2 > 0:
-        # the dominant kernel is k_step2 (two steps per launch, one read and one
+    # every FP32 workload above is a cavity or channel that the library advances
+    # two steps per launch unless its tuning says otherwise
+    two = w["storage"] == 0 and b.get_tuning()["temporal"] != 0
+    if two:
+        # the dominant kernel is k_sweep (two steps per launch, one read and one
         # write of the populations); its launch time from two runs of 2m + 1
         # steps (m two-step launches and one single step each)
         seg2 = []
@@ -556,7 +559,7 @@ def main():
                 b.run(steps)
                 tot.append(b.timing()[0] * steps)
             seg2.append((tot[1] - tot[0]) / 100)
-        kernel = {"name": "k_step2", "steps_per_launch": 2, "launch_ms": statistics.median(seg2),
+        kernel = {"name": "k_sweep", "steps_per_launch": 2, "launch_ms": statistics.median(seg2),
                   "launch_ms_samples": [round(x, 5) for x in seg2]}
     else:
         kernel = {"name": "k_step", "steps_per_launch": 1, "launch_ms": dev_ms}
@@ -593,7 +596,7 @@ def main():
         "data": "synthetic (lattice initialised at rest, rho = 1)",
         "config": {"workload": w["desc"], "nx": w["nx"], "ny": w["ny"], "nz": w["nz"], "nodes": n,
                    "tuning": dict(b.get_tuning(), ms_per_step=tuned_ms, autotuned=not args.no_autotune, step2_height=h2,
-                                  graph_replay=h2 == 0 and args.graph_steps > 0 and min(segs, default=0) >= args.graph_steps),
+                                  graph_replay=not two and args.graph_steps > 0 and min(segs, default=0) >= args.graph_steps),
                    "device": name, "cus": cus},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic_from_profiles(args.workload, kn),

@@ -204,17 +204,18 @@ typedef struct nflow_tuning {
   int xcd_order;   /* 1: each XCD receives a contiguous range of work items */
   int persistent;  /* 0: one workgroup per work item; k > 0: k workgroups per CU, grid-stride */
   int graph_steps; /* steps per captured graph (even), 0 = no graph */
-  /* Two steps per launch for a batch of one FP32 cavity or channel lattice
-   * without solid nodes (other batches ignore this): x-z tiles of 256 x 8 nodes swept along
-   * y in chunks of H planes, with results bit for bit those of one step per
-   * launch.  A run of odd length ends with a single step; one of even length
-   * ends with a two-step launch, which a read-back of its state re-runs as two
-   * single steps (launches only), unless the previous run's state was read
-   * back: then it ends with two single steps.  H > 0: that chunk
-   * height; -1 (the default): chosen by the library from an estimate of the
-   * launch time at heights 8 to 64, on where the estimate beats one step per
-   * launch (cavities from about 176^3 up, channels of 128 x 128 cross-section
-   * from 256 long); 0: one step per launch.  The autotuner times it. */
+  /* Two steps per launch for FP32 cavities and channels without solid nodes
+   * (other batches ignore this), in x-z tiles swept along y in chunks of H
+   * planes, with results bit for bit those of one step per launch.  A run of
+   * odd length ends with a single step; one of even length ends with a
+   * two-step launch, which a read-back of its state re-runs as two single
+   * steps (launches only), unless the previous run's state was read back:
+   * then it ends with two single steps.  H > 0: that chunk height (batches of
+   * one lattice; others take one step per launch); -1 (the default): tiles
+   * and heights chosen by the library from an estimate of the launch time, on
+   * where that beats one step per launch (from about 56^3 nodes up; batches
+   * of several lattices by the sum of theirs); 0: one step per launch.  The
+   * autotuner times it. */
   int temporal;
   double ms_per_step; /* filled by the autotuner */
 } nflow_tuning;
@@ -227,8 +228,11 @@ int nflow_batch_get_tuning(nflow_batch* b, nflow_tuning* t);
 /* launch shape of a single-lattice solver (it is a batch of one; no
  * reference counterpart): the same fields and rules as for a batch */
 int nflow_set_tuning(nflow_solver* s, const nflow_tuning* t);
-/* chunk height the batch's runs use for two steps per launch under its tuning
- * (temporal = -1 resolved), 0 when every launch is a single step */
+/* chunk height that the batch's tuning names for two steps per launch: its
+ * temporal where that is > 0, for -1 the estimate for tiles of 256 x 8 nodes,
+ * 0 where that estimate finds one step per launch faster (and for batches of
+ * several lattices, 16-bit storage and solid nodes).  With -1 a run may use
+ * other tiles and heights than this, also where it is 0. */
 int nflow_batch_step2_height(nflow_batch* b);
 int nflow_batch_run(nflow_batch* b, int nsteps);
 int nflow_batch_synchronize(nflow_batch* b);

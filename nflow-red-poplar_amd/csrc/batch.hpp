@@ -60,6 +60,11 @@ class Batch {
   size_t d_items_cap = 0;
   int nitems = 0;
   int grid = 0;
+  // work list of two-step launches (nsweep = 0: one step per launch)
+  SweepItem* d_sweep = nullptr;
+  size_t d_sweep_cap = 0;
+  int nsweep = 0;
+  bool sweep_channel = false, sweep_runs = false;
   bool tables_dirty = true;
   bool masked = false;  // some lattice has solid nodes: step with the masked kernel
   bool sr_any = false;  // some lattice rounds its 16-bit stores stochastically
@@ -103,8 +108,8 @@ class Batch {
   int launch_steps(int nsteps);  // enqueue only
   // After a run that ended with a two-step launch, re-run that launch as two
   // single steps from the state it read (still in buf[cur ^ 1]), so that
-  // buf[cur ^ 1] holds the previous step's state again; the same values, bit
-  // for bit.  Kernel launches only: no allocation.  No-op otherwise.
+  // buf[cur ^ 1] holds the previous step's state again in every lattice; the
+  // same values, bit for bit.  Kernel launches only: no allocation.  No-op otherwise.
   int settle_pair();
   int run(int nsteps);           // enqueue with timing events
   int synchronize();
@@ -120,9 +125,12 @@ class Batch {
   int node_types(int idx, int* type, int* dirstate);
   int autotune(int trial_steps, nflow_tuning* out);
   int set_tuning(const nflow_tuning& t);
-  // y-chunk height of two-step launches for this batch under `t` (tuning by
-  // default), resolving temporal = -1; 0: one step per launch
+  // y-chunk height that `t` (tuning by default) names for two-step launches of
+  // 256 x 8 node tiles, resolving temporal = -1 by an estimate for those; 0:
+  // none
   int step2_height(const nflow_tuning* t = nullptr) const;
+  // work list of two-step launches under `t`, empty for one step per launch
+  std::vector<SweepItem> sweep_items(const nflow_tuning& t) const;
   void destroy_graphs();
   long long total_nodes() const;
   size_t device_bytes() const;

@@ -285,9 +285,10 @@ __device__ inline int node_type(const LatticeDev& L, int x, int y, int z) {
 // node at x - e_x, so its index is one of three per-node bases (x - 1, x,
 // x + 1) plus a wave-uniform term, one add per population in place of a full
 // index computation.
-template <class St, bool MASK, class Acc, bool RUNS = false>
-__device__ inline void pull(const LatticeDev& L, const Acc& in, uint32_t n, uint32_t nr, int x, int y, int z,
-                            float f[Q]) {
+// take(q, v) receives each stored element.
+template <class St, bool MASK, class Acc, bool RUNS, class Take>
+__device__ __forceinline__ void pull_each(const LatticeDev& L, const Acc& in, uint32_t n, uint32_t nr, int x, int y,
+                                          int z, Take take) {
   using T = typename St::T;
   const bool xlo = x == 0, xhi = x == L.nx - 1;
   const bool ylo = y == 0, yhi = y == L.ny - 1;
@@ -324,8 +325,14 @@ __device__ inline void pull(const LatticeDev& L, const Acc& in, uint32_t n, uint
       }
       idx = out ? pidx<T>(OPP[q], nr, ps) : pidx<T>(q, (uint32_t)((int)nr - off), ps);
     }
-    f[q] = load_f<St>(in.get(idx), q);
+    take(q, in.get(idx));
   }
+}
+
+template <class St, bool MASK, class Acc>
+__device__ inline void pull(const LatticeDev& L, const Acc& in, uint32_t n, uint32_t nr, int x, int y, int z,
+                            float f[Q]) {
+  pull_each<St, MASK, Acc, false>(L, in, n, nr, x, y, z, [&](int q, typename St::T v) { f[q] = load_f<St>(v, q); });
 }
 
 // Inputs of the inlet / outlet rules from the previous step's side planes:
@@ -394,11 +401,11 @@ __device__ inline void boundary(const LatticeDev& L, const SideIn& si, int x, in
   }
 }
 
-template <class St, bool MASK, class Acc, bool RUNS = false>
+template <class St, bool MASK, class Acc>
 __device__ inline void gather(const LatticeDev& L, const Acc& in, const float* __restrict__ side, uint32_t n,
                               uint32_t nr, int x, int y, int z, float f[Q]) {
   const SideIn si = side_inputs(L, side, x, y, z);
-  pull<St, MASK, Acc, RUNS>(L, in, n, nr, x, y, z, f);
+  pull<St, MASK, Acc>(L, in, n, nr, x, y, z, f);
   boundary(L, si, x, y, z, f);
 }
 
@@ -710,242 +717,273 @@ __global__ void __launch_bounds__(256) k_advance(const LatticeDev* __restrict__ 
 #endif
 
 // ---------------------------------------------------------------------------
-// Two time steps per launch (a cavity or channel lattice without solid nodes).
+// Two time steps per launch (FP32 cavity and channel lattices without solid
+// nodes): k_sweep.
 //
-// A workgroup owns a TX x TZ tile of the x-z plane and a range [ya, yb) of y
-// planes, and sweeps it in y.  TX spans whole x rows of the benchmark sizes:
-// the pulls of a 128-byte line granularity make every x edge of a tile cost
-// about 28 extra lines per row, so the tile has none where nx <= TX.  Thread
-// t owns K nodes of column x0 + t % TX, stacked in z.  For each plane yi:
+// A workgroup owns a tile of tx x tz nodes of the x-z plane, one per thread,
+// and a range [ya, yb) of y planes, and sweeps it in y.  For each plane yi:
 //   1. the first of the two steps (pull from buf[p] with the boundary rules,
 //      collision) on the own nodes and on the halo around the tile (the rows
-//      z0 - 1 and z0 + TZ, and the columns x0 - 1 and x0 + TX where they are
-//      inside the box), spread over the threads; populations that cross to
-//      another x-z column go to LDS (from the halo rows only the 5 that cross
-//      into the tile in z); the own node's rest population, e = (0, +-1, 0)
-//      and the bounce-back of its links that leave the box go straight to its
-//      registers;
-//   2. each thread collects the crossing populations its nodes pull from
-//      plane yi: e_y = -1 ones for plane yi - 1, e_y = 0 ones for plane yi,
-//      e_y = +1 ones for plane yi + 1;
-//   3. the second step of plane yi - 1, whose 19 pulled values are now
-//      complete, stored to buf[p ^ 1].
-// The partial pulls of planes yi and yi + 1 stay in registers.
+//      z0 - 1 and z0 + tz, and the columns x0 - 1 and x0 + tx where they are
+//      inside the box), one halo node per thread; the populations that cross
+//      to another x-z column go to LDS (from the halo only those that cross
+//      into the tile), the own node's rest population and e = (0, +-1, 0)
+//      stay in its registers;
+//   2. the loads of the own nodes' next plane are issued, so that they are in
+//      flight during the rest of this plane;
+//   3. after the plane's one barrier each thread collects what its node pulls
+//      from plane yi: e_y = -1 populations for plane yi - 1, whose 19 pulled
+//      values are now complete and take the second step to buf[p ^ 1]; then
+//      e_y = 0 ones for plane yi and e_y = +1 ones for plane yi + 1 (19
+//      registers in all between planes).
+// The exchange has two halves, for even and odd planes: a wave that runs ahead
+// fills the one while others still read the other, so a plane needs one
+// barrier, and what a node left in the other half one plane ago is still
+// there for the links of plane yi - 1 that bounce back.
 //
-// Built for FP32 storage.  Per node and step the arithmetic and the stored
-// values are those of k_step (both compiled with -ffp-contract=on, so an FMA
-// never spans statements and the collision rounds the same in either kernel),
-// so two launches of k_step and one of k_step2 give the same state bit for
-// bit; the memory traffic of the pair is one read and one write of the
-// populations (plus the halo) instead of two of each.  The intermediate state
-// never reaches memory, so the launch before a read-back must be a k_step
-// (the export streams the state the last launch read): a run that ends with
-// a k_step2 is settled by re-running it as two k_step launches from the state
-// it read, which it leaves untouched.
+// Per node and step the arithmetic and the stored values are those of k_step
+// (both compiled with -ffp-contract=on, so an FMA never spans statements and
+// the collision rounds the same in either kernel), so two launches of k_step
+// and one of k_sweep give the same state bit for bit; the memory traffic of
+// the pair is one read and one write of the populations (plus the halo)
+// instead of two of each.  The intermediate state never reaches memory, so the
+// launch before a read-back must be a k_step (the export streams the state the
+// last launch read): a run that ends with a k_sweep is settled by re-running
+// it as two k_step launches from the state it read, which it leaves untouched.
+//
+// Why this shape.  One node per thread leaves registers for the prefetch (a
+// sweep with two nodes per thread and no room for one, which this kernel
+// replaced, waited for its gathers with no loads in flight during the second
+// steps and barriers), and tiles of whole rows of any width, 1024 / tx rows
+// high, keep the lanes busy where tiles of a fixed 256 x 8 nodes left most
+// idle.  Measured (us per step, one step per launch / the two-node sweep /
+// this one): 256^3 432 / 254 / 229, 4.5 TB/s x 2; 128^3 55 / 55 / 33.8; 96^3
+// 25.6 / 25.6 / 16.6; 101 x 67 x 83 19.1 / 19.1 / 13.6; 512^3 3701 / 2067 /
+// 1816; channels 512 x 128 x 128 215 / 153 / 132 and 676 x 128 x 128 298 /
+// 268 / 232.  At 256^3 a plane takes 6.9 us, against 6.3 us for its bytes at
+// the layout's copy rate.  16-bit storage does not gain: there the collision,
+// the conversions and the halo's share of them bind (256^3 FP16 with
+// stochastic rounding 244 us against 216 for one step per launch).
 // ---------------------------------------------------------------------------
-namespace step2 {
-// Slot of crossing population q (e_x or e_z non-zero) in an LDS row: the 5
-// with e_z = -1 first (3, 7, 8, 15, 17), then the 6 with e_z = 0, then the 5
-// with e_z = +1 (4, 9, 10, 16, 18); -1: the own column keeps it (rest, e =
-// (0, +-1, 0)).  The rows of the tile are stored one after another, the halo
-// row z0 - 1 before them with only its e_z = +1 slots (the ones pulled into
-// the tile) and the halo row z0 + TZ after them with only its e_z = -1 slots,
-// so that every access is one per-thread base plus a constant.
-constexpr int CIX[Q] = {-1, 5, 6, 0, 11, -1, -1, 1, 2, 12, 13, 7, 8, 9, 10, 3, 14, 4, 15};
-constexpr int NC = 16;
+namespace sweep {
+// Slots of the crossing populations (e_x or e_z non-zero): those with e_z = 0
+// or -1 first (11, own node at element lz * WX + lx + 1 of the slot), then
+// those with e_z = +1 (5, own node one row further on, behind the tile row
+// -1); -1: the own column keeps it.
 constexpr int QUP = 5, QDN = 6;  // e = (0, +1, 0), (0, -1, 0)
-
-template <int TX_, int TZ_, int NT_>
-struct Geo {
-  static constexpr int TX = TX_, TZ = TZ_, NT = NT_, WX = TX + 2;
-  static constexpr int RP = NT / TX;  // x rows per pass of the threads
-  static constexpr int K = TZ / RP;   // own nodes per thread
-  static_assert(NT % TX == 0 && TZ % RP == 0, "whole rows per thread pass");
-  static_assert(TX % 64 == 0, "a wave within one row group");
-  // Tile row of own node j of row group r.  The halo rows of a tile pull the
-  // same elements as the edge rows of the neighbouring tiles, which run on the
-  // same XCD; the halo goes to the first row groups, so the edge rows (0 and
-  // TZ - 1) go to row groups without halo work, as their first node, and are
-  // computed in the same pass of the plane as the neighbours' halo rows: the
-  // second load of those lines then finds them in L2 (measured at 256^3:
-  // 302.4 -> 297.0 us per step).
-  __device__ static constexpr int row(int r, int j) {
-    if constexpr (TZ == 8 && RP == 4 && K == 2) {
-      constexpr int R[4][2] = {{1, 2}, {3, 4}, {0, 5}, {7, 6}};
-      return R[r][j];
-    }
-    return r * K + j;
+constexpr int slot_of(int q) {
+  if (EX[q] == 0 && EZ[q] == 0) return -1;
+  int c = 0;
+  for (int k = 0; k < Q; ++k) {
+    if (EX[k] == 0 && EZ[k] == 0) continue;
+    const bool up = EZ[k] > 0, me = EZ[q] > 0;
+    if (up < me || (up == me && (EZ[k] < EZ[q] || (EZ[k] == EZ[q] && k < q)))) ++c;
   }
-  // LDS element of slot c of row zs (-1 .. TZ) at column-frame x xs
-  static constexpr int LN = (TZ * NC + 10) * WX;
-  __device__ static constexpr int lidx(int zs, int c, int xs) { return ((zs + 1) * NC + c - 11) * WX + xs; }
-};
-}  // namespace step2
+  return c;
+}
+constexpr int S1 = SWEEP_SLOT1, S0 = SWEEP_SLOT0;  // elements of a slot with e_z != 0, = 0
+// slots 0-4: e_z = -1; 5-10: e_z = 0; 11-15: e_z = +1
+constexpr int base_of(int c) { return c <= 5 ? c * S1 : c <= 11 ? 5 * S1 + (c - 5) * S0 : 5 * S1 + 6 * S0 + (c - 11) * S1; }
+constexpr int LN = 10 * S1 + 6 * S0;
+}  // namespace sweep
 
-// CH: a channel lattice (velocity inlet at x = 0, pressure outlet at x =
-// nx - 1).  The second step's inlet and outlet rules read the first step's
-// rho at x = 1 and u at x = nx - 1 and nx - 2 on the same plane; the first
-// step leaves them in LDS (two plane slots), where k_step would have written
-// the side records, and the second step writes the side records the next
-// launch reads.
-// RUNS: nx is a multiple of the 64-node block, and the pulls index donors
-// from three per-node bases (pull<..., RUNS>).
-template <class St, class G, bool CH, bool RUNS>
-__global__ void __launch_bounds__(G::NT) k_step2(LatticeDev L, int parity, int H, int ntx, int ntz) {
-  static_assert(!St::shifted, "two steps per launch are built for FP32 storage");
-  using namespace step2;
+// CH: some lattice of the launch is a channel (velocity inlet at x = 0, pressure
+// outlet at x = nx - 1).  Its rules read the previous step's rho at x = 1 and u
+// at x = nx - 1 and nx - 2: the first step takes them from the side records,
+// fetched one plane ahead, the second from what the first left in LDS, and the
+// second step writes the records the next launch reads.
+// RUNS: nx is a multiple of the 64-node block in every lattice of the launch
+// (pull<..., RUNS>).
+template <class St, bool CH, bool RUNS>
+__global__ void __launch_bounds__(SWEEP_NT) k_sweep(const LatticeDev* __restrict__ lats,
+                                                    const SweepItem* __restrict__ items, int parity) {
+  using namespace sweep;
   using T = typename St::T;
-  constexpr int TX = G::TX, TZ = G::TZ, NT = G::NT, K = G::K;
-  // crossing populations of the own rows (with the x - 1 and x + TX columns)
-  // and of the halo rows z0 - 1 (e_z = +1 ones) and z0 + TZ (e_z = -1 ones)
-  __shared__ T cross[G::LN];
-  // channel: the first step's rho(x = 1), u(nx - 1), u(nx - 2) of each tile
-  // row, for planes of even and odd y
-  __shared__ float sidein[CH ? 2 : 1][TZ][8];
-  int bt = blockIdx.x;
-  // workgroups are dispatched to the 8 XCDs round-robin: give each XCD a
-  // contiguous range of tiles, so that neighbours share their halo in L2
-  if ((gridDim.x & 7u) == 0) bt = (bt & 7) * (int)(gridDim.x >> 3) + (bt >> 3);
-  const int tx = bt % ntx, tz = (bt / ntx) % ntz, ch = bt / (ntx * ntz);
-  const int x0 = tx * TX, z0 = tz * TZ, ya = ch * H, yb = min(L.ny, ya + H);
+  __shared__ T cross[2 * LN];
+  // channel: the first step's rho(x = 1), u(nx - 1), u(nx - 2) and the inlet
+  // velocity of each tile row (planes y mod 4), for the second step's rules
+  __shared__ float sidein[CH ? 4 : 1][CH ? SWEEP_ROWS : 1][8];
+  // channel: the first step's inputs, from the side records of the previous
+  // launch, of the tile's rows and the two around it (planes y mod 2)
+  __shared__ float sidepre[CH ? 2 : 1][CH ? SWEEP_ROWS + 2 : 1][8];
+  const SweepItem it = items[blockIdx.x];
+  if (it.h == 0) return;  // padding of the work list
+  const LatticeDev& L = lats[it.lat];
+  const int x0 = it.x0, z0 = it.z0, ya = it.ya, yb = min(L.ny, it.ya + it.h);
+  const int txn = min(it.tx, L.nx - x0), tzn = min(it.tz, L.nz - z0), WX = txn + 2;
   const int p = parity ^ L.parity0;
   // The buffers are viewed from the block of the lowest plane the workgroup
   // reads (y = ya - 2, pulled by the first step on plane ya - 1): 32-bit
-  // element indices whatever the lattice size.  Loads without the
-  // non-temporal hint: the halo rows, and the planes on either side of a y
-  // chunk, are loaded again by the neighbouring tile or chunk, and then find
-  // them in L2 (measured per launch, 256^3 cavity: 604 -> 564 us; 512 x 128
-  // x 128 channel: 372 -> 356 us).  The stores keep it.
+  // offsets whatever the lattice size.  Loads without the non-temporal hint:
+  // the halo rows, and the planes on either side of a y chunk, are loaded
+  // again by the neighbouring tile or chunk, and then find them in L2.
   constexpr uint32_t B = 256 / sizeof(T);
   const uint32_t bn = ((uint32_t)max(ya - 2, 0) * (uint32_t)L.nxz) & ~(B - 1);
   const GPops<T, false> in{static_cast<T*>(L.buf[p]) + window<T>(bn)};
   const GPops<T> out{static_cast<T*>(L.buf[p ^ 1]) + window<T>(bn)};
   const int t = threadIdx.x;
-  // own nodes: (x0 + lx, z0 + zrow[j]), j < K; the row group rg is the same
-  // for a whole wave
-  const int lx = t % TX, rg = __builtin_amdgcn_readfirstlane(t / TX);
-  int zrow[K];  // tile row of own node j
-#pragma unroll
-  for (int j = 0; j < K; ++j) zrow[j] = G::row(rg, j);
-  const int ox = x0 + lx;
-  const bool xin = ox < L.nx, xlo = ox == 0, xhi = ox == L.nx - 1;
-  // halo nodes of the tile: row z0 - 1, row z0 + TZ (x from xa to xb), column
-  // x0 - 1, column x0 + TX (z0 .. z0 + tzn - 1), each where inside the box
-  const int xa = max(x0 - 1, 0), xb = min(x0 + TX, L.nx - 1), rowlen = xb - xa + 1;
-  const int tzn = min(TZ, L.nz - z0);
-  const int nlo = z0 > 0 ? rowlen : 0, nhi = z0 + TZ < L.nz ? rowlen : 0;
-  const int nxl = x0 > 0 ? tzn : 0, nxr = x0 + TX < L.nx ? tzn : 0;
-  const int nhalo = nlo + nhi + nxl + nxr;
-  // element index base of node (x, y, z) in the window
+  // own node: (x0 + lx, z0 + lz)
+  const int lz = t / txn, lx = t - lz * txn;
+  const bool own_in = lz < tzn;
+  int ox = x0 + lx, oz = z0 + lz;
+  // this thread's halo node: row z0 - 1, row z0 + tzn (x from xa to xb),
+  // column x0 - 1, column x0 + txn, each where inside the box
+  const int xa = max(x0 - 1, 0), xb = min(x0 + txn, L.nx - 1), rowlen = xb - xa + 1;
+  const int nlo = z0 > 0 ? rowlen : 0, nhi = z0 + tzn < L.nz ? rowlen : 0;
+  const int nxl = x0 > 0 ? tzn : 0, nxr = x0 + txn < L.nx ? tzn : 0;
+  const bool halo_in = t < nlo + nhi + nxl + nxr;
+  int hx, hz, kind;  // kind 0: row z0 - 1, 1: row z0 + tzn, 2: column x0 - 1, 3: column x0 + txn
+  if (t < nlo) { hx = xa + t; hz = z0 - 1; kind = 0; }
+  else if (t < nlo + nhi) { hx = xa + (t - nlo); hz = z0 + tzn; kind = 1; }
+  else if (t < nlo + nhi + nxl) { hx = x0 - 1; hz = z0 + (t - nlo - nhi); kind = 2; }
+  else { hx = x0 + txn; hz = z0 + (t - nlo - nhi - nxl); kind = 3; }
+  // index of node (x, y, z) in the window
   auto node = [&](int x, int y, int z) {
     return (uint32_t)x + (uint32_t)L.nx * ((uint32_t)z + (uint32_t)L.nz * (uint32_t)y) - bn;
   };
-  // first step on node (x, yi, z): e = the stored values, g = them as the
-  // next step reads them back
-  auto step1 = [&](int x, int yi, int z, T e[Q], float g[Q]) {
-    const uint32_t n = node(x, yi, z);
+  const int o0 = own_in ? lz * WX + lx : 0;  // own element of a slot, less one
+  // the halo node's element of its slots (rows: e_z = +1 resp. -1 slots;
+  // columns: e_z <= 0 slots, one row further on for e_z = +1)
+  const int h0 = (kind == 0 ? 0 : (kind == 1 ? tzn : hz - z0) * WX) + hx - x0 + 1;
+  T raw[Q];
+  auto issue = [&](int x, int y, int z, T r[Q]) {
+    const uint32_t n = node(x, y, z);
+    pull_each<St, false, decltype(in), RUNS>(L, in, n, n, x, y, z, [&](int q, T v) { r[q] = v; });
+  };
+  // the first step on a node whose pulled values are r: e = the stored values
+  auto step1 = [&](const T r[Q], int x, int yi, int z, T e[Q]) {
+    float g[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) g[q] = load_f<St>(r[q], q);
     if constexpr (CH) {
-      gather<St, false, decltype(in), RUNS>(L, in, L.side[p], n, n, x, yi, z, g);
+      const float* sp = sidepre[yi & 1][z - z0 + 1];
+      SideIn si = {};
+      if (x == 0) {
+        si.v[0] = sp[0];
+        si.v[1] = sp[1];
+      } else if (x == L.nx - 1) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) si.v[k] = sp[2 + k];
+      }
+      boundary(L, si, x, yi, z, g);
       float mac[4];
       relax<false>(L, g, nullptr, x, yi, z, mac);
-      if (z >= z0 && z < z0 + TZ) {  // rows of the tile: what its second step reads
-        float* r = sidein[yi & 1][z - z0];
-        if (x == 1) r[0] = mac[0];
-        if (x == L.nx - 1) { r[1] = mac[1]; r[2] = mac[2]; r[3] = mac[3]; }
-        if (x == L.nx - 2) { r[4] = mac[1]; r[5] = mac[2]; r[6] = mac[3]; }
+      if (z >= z0 && z < z0 + tzn) {
+        float* rr = sidein[yi & 3][z - z0];
+        if (x == 0) rr[7] = si.v[1];
+        if (x == 1) rr[0] = mac[0];
+        if (x == L.nx - 1) { rr[1] = mac[1]; rr[2] = mac[2]; rr[3] = mac[3]; }
+        if (x == L.nx - 2) { rr[4] = mac[1]; rr[5] = mac[2]; rr[6] = mac[3]; }
       }
     } else {
-      pull<St, false, decltype(in), RUNS>(L, in, n, n, x, yi, z, g);
-      boundary(L, SideIn{{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f}}, x, yi, z, g);
+      if (yi == L.ny - 1) boundary(L, SideIn{{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f}}, x, yi, z, g);
       relax<false>(L, g, nullptr, x, yi, z);
     }
 #pragma unroll
-    for (int q = 0; q < Q; ++q) {
-      e[q] = St::enc(g[q] - shift_of<St>(q));
-      g[q] = load_f<St>(e[q], q);
-    }
+    for (int q = 0; q < Q; ++q) e[q] = St::enc(g[q] - shift_of<St>(q));
   };
-
-  // Pulled values of own node j: fp on plane yi - 1 (complete but for the
-  // e_y = -1 crossing links from plane yi), fc on plane yi (so far its e_y =
-  // +1 links), fn the e_y = +1 links of plane yi + 1.
-  float fp[K][Q], fc[K][Q], fn[K][Q];
-#pragma unroll
-  for (int j = 0; j < K; ++j)
-#pragma unroll
-    for (int q = 0; q < Q; ++q) fp[j][q] = fc[j][q] = fn[j][q] = 0.0f;
-  // does the link of q at own node j on plane y leave the box?
-  auto gone = [&](int q, int j, int y) {
-    const int oz = z0 + zrow[j];
-    return (EX[q] > 0 && xlo) || (EX[q] < 0 && xhi) || (EY[q] > 0 && y == 0) || (EY[q] < 0 && y == L.ny - 1) ||
-           (EZ[q] > 0 && oz == 0) || (EZ[q] < 0 && oz == L.nz - 1);
+  // does the link of q at the own node on plane y leave the box?
+  auto gone = [&](int q, int y) {
+    return (EX[q] > 0 && ox == 0) || (EX[q] < 0 && ox == L.nx - 1) || (EY[q] > 0 && y == 0) ||
+           (EY[q] < 0 && y == L.ny - 1) || (EZ[q] > 0 && oz == 0) || (EZ[q] < 0 && oz == L.nz - 1);
   };
+  // Pulled values: fp on plane yi - 1 (complete but for the e_y = -1 links
+  // from plane yi), fc on plane yi (so far its e_y = +1 links), fn the
+  // e_y = +1 links of plane yi + 1.
+  T fp[Q], fc[Q], fn[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) fp[q] = fc[q] = fn[q] = (T)0.0f;
+  // side records: thread t holds float t mod 8 of row z0 - 1 + t / 8
+  const int sz = z0 - 1 + (t >> 3);
+  const bool side_in = CH && L.casetype != CASE_CAVITY && t < (tzn + 2) * 8 && sz >= 0 && sz < L.nz;
+  auto side_load = [&](int y) {
+    const int k = t & 7;
+    const int at = k < 2 ? SIDE_RHO + k : k < 5 ? SIDE_U0 + k - 2 : SIDE_U1 + k - 5;
+    return ((gptr<const float>)L.side[p])[(size_t)(y * L.nz + sz) * SIDE_REC + at];
+  };
+  if constexpr (CH) {
+    if (side_in) sidepre[max(ya - 1, 0) & 1][t >> 3][t & 7] = side_load(max(ya - 1, 0));
+    __syncthreads();
+  }
+  if (own_in) issue(ox, max(ya - 1, 0), oz, raw);
   for (int yi = ya - 1; yi <= yb; ++yi) {
     const bool plane = yi >= 0 && yi < L.ny;
+    // element of the own node in this plane's half of the exchange, less one;
+    // opaque, so that the addresses and wall tests derived from it and from
+    // the coordinates are formed in the loop and not kept across it
+    int c0 = (yi & 1) * LN + o0, ch = (yi & 1) * LN + h0;
+    asm volatile("" : "+v"(c0), "+v"(ch), "+v"(ox), "+v"(oz));
     if (plane) {
-      for (int h = t; h < nhalo; h += NT) {  // halo
-        int x, z, kind;  // kind 0: row z0 - 1, 1: row z0 + TZ, 2: a column
-        if (h < nlo) { x = xa + h; z = z0 - 1; kind = 0; }
-        else if (h < nlo + nhi) { x = xa + (h - nlo); z = z0 + TZ; kind = 1; }
-        else if (h < nlo + nhi + nxl) { x = x0 - 1; z = z0 + (h - nlo - nhi); kind = 2; }
-        else { x = x0 + TX; z = z0 + (h - nlo - nhi - nxl); kind = 2; }
+      T rh[Q];
+      float sv = 0.0f;
+      if constexpr (CH)
+        if (side_in && yi + 1 < L.ny) sv = side_load(yi + 1);
+      if (halo_in) issue(hx, yi, hz, rh);
+      if (own_in) {
         T e[Q];
-        float g[Q];
-        step1(x, yi, z, e, g);
-        if (kind == 2) {
+        step1(raw, ox, yi, oz, e);
+        const int c1 = c0 + WX;
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+          if (slot_of(q) >= 0) cross[(EZ[q] > 0 ? c1 : c0) + base_of(slot_of(q)) + 1] = e[q];
+        fc[0] = e[0];
+        fn[QUP] = e[QUP];
+        fp[QDN] = e[QDN];
+        fc[QUP] = yi == 0 ? e[QDN] : fc[QUP];
+      }
+      asm volatile("" ::: "memory");  // the halo node's arithmetic after the own node's: registers
+      if (halo_in) {
+        T e[Q];
+        step1(rh, hx, yi, hz, e);
+        if (kind == 0) {
 #pragma unroll
           for (int q = 0; q < Q; ++q)
-            if (CIX[q] >= 0) cross[G::lidx(z - z0, CIX[q], x - x0 + 1)] = e[q];
+            if (EZ[q] > 0) cross[ch + base_of(slot_of(q))] = e[q];
+        } else if (kind == 1) {
+#pragma unroll
+          for (int q = 0; q < Q; ++q)
+            if (EZ[q] < 0) cross[ch + base_of(slot_of(q))] = e[q];
+        } else if (kind == 2) {
+#pragma unroll
+          for (int q = 0; q < Q; ++q)
+            if (EX[q] > 0) cross[(EZ[q] > 0 ? ch + WX : ch) + base_of(slot_of(q))] = e[q];
         } else {
 #pragma unroll
           for (int q = 0; q < Q; ++q)
-            if (EZ[q] != 0 && (EZ[q] > 0) == (kind == 0)) cross[G::lidx(z - z0, CIX[q], x - x0 + 1)] = e[q];
+            if (EX[q] < 0) cross[(EZ[q] > 0 ? ch + WX : ch) + base_of(slot_of(q))] = e[q];
         }
       }
-    }
-#pragma unroll
-    for (int j = 0; j < K; ++j) {  // own nodes
-      const int oz = z0 + zrow[j];
-      float g[Q];
-      if (plane && xin && oz < L.nz) {
-        T e[Q];
-        step1(ox, yi, oz, e, g);
-#pragma unroll
-        for (int q = 0; q < Q; ++q)
-          if (CIX[q] >= 0) cross[G::lidx(zrow[j], CIX[q], lx + 1)] = e[q];
-      } else {
-#pragma unroll
-        for (int q = 0; q < Q; ++q) g[q] = 0.0f;
-      }
-      fc[j][0] = g[0];
-      fn[j][QUP] = g[QUP];
-      fp[j][QDN] = yi - 1 == L.ny - 1 ? fp[j][QDN] : g[QDN];  // leaves only from plane ny - 1
-      fc[j][QDN] = gone(QDN, j, yi) ? g[QUP] : 0.0f;
-      fc[j][QUP] = gone(QUP, j, yi) ? g[QDN] : fc[j][QUP];
+      asm volatile("" ::: "memory");  // and the next plane's loads after both
+      if constexpr (CH)
+        if (side_in) sidepre[(yi + 1) & 1][t >> 3][t & 7] = sv;
+      if (own_in && yi < yb && yi + 1 < L.ny) issue(ox, yi + 1, oz, raw);
     }
     __syncthreads();
-    // crossing population q pulled by own node j from plane yi
-    auto pulled = [&](int q, int j) {
-      return load_f<St>(cross[G::lidx(zrow[j] - EZ[q], CIX[q], lx + 1 - EX[q])], q);
-    };
-    // own node j's crossing population q after the first step on plane yi
-    auto own = [&](int q, int j) { return load_f<St>(cross[G::lidx(zrow[j], CIX[q], lx + 1)], q); };
     const int yf = yi - 1;
-#pragma unroll
-    for (int j = 0; j < K; ++j) {  // second step on plane yf
-      const int oz = z0 + zrow[j];
+    if (own_in) {
+      // crossing population q pulled from plane yi, and the own node's
+      const int c1 = c0 + WX;
+      auto pulled = [&](int q) { return cross[(EZ[q] < 0 ? c1 : c0) + base_of(slot_of(q)) + 1 - EX[q]]; };
+      auto own = [&](int q) { return cross[(EZ[q] > 0 ? c1 : c0) + base_of(slot_of(q)) + 1]; };
+      // the own node's on plane yf, still in the other half of the exchange
+      const int d0 = c0 + (yi & 1 ? -LN : LN), d1 = d0 + WX;
+      auto before = [&](int q) { return cross[(EZ[q] > 0 ? d1 : d0) + base_of(slot_of(q)) + 1]; };
 #pragma unroll
       for (int q = 0; q < Q; ++q)
-        if (CIX[q] >= 0 && EY[q] < 0) fp[j][q] = gone(q, j, yf) ? fp[j][q] : pulled(q, j);
-      if (xin && oz < L.nz && yf >= ya && yf < yb) {
+        if (slot_of(q) >= 0 && EY[q] < 0) fp[q] = gone(q, yf) ? before(OPP[q]) : pulled(q);
+      if (yf == L.ny - 1) fp[QDN] = fc[QUP];
+      if (yf >= ya && yf < yb) {
         const uint32_t n = node(ox, yf, oz);
-        SideIn si = {{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f}};
-        if constexpr (CH) {  // side_inputs(), from the first step's values
+        float g[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) g[q] = load_f<St>(fp[q], q);
+        if constexpr (CH) {
+          SideIn si = {{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f}};
           if ((ox == 0 || ox == L.nx - 1) && !(yf == 0 || yf == L.ny - 1 || oz == 0 || oz == L.nz - 1)) {
-            const float* r = sidein[yf & 1][zrow[j]];
+            const float* r = sidein[yf & 3][lz];
             if (ox == 0) {
               si.v[0] = r[0];
-              si.v[1] = ((gptr<const float>)L.side[p])[(size_t)(yf * L.nz + oz) * SIDE_REC + SIDE_UIN];
+              si.v[1] = r[7];
             } else {
               si.v[0] = r[1];
               si.v[1] = r[2];
@@ -955,34 +993,32 @@ __global__ void __launch_bounds__(G::NT) k_step2(LatticeDev L, int parity, int H
               si.v[5] = r[6];
             }
           }
+          boundary(L, si, ox, yf, oz, g);
+        } else {
+          if (yf == L.ny - 1) boundary(L, SideIn{{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f}}, ox, yf, oz, g);
         }
-        boundary(L, si, ox, yf, oz, fp[j]);
-        relax_and_store<St, false, CH>(L, fp[j], out, L.side[p ^ 1], n, ox, yf, oz, 0u);
+        relax_and_store<St, false, CH>(L, g, out, L.side[p ^ 1], n, ox, yf, oz, 0u);
+      }
+      asm volatile("" ::: "memory");  // the other populations are read after the second step
+      if (plane) {
+#pragma unroll
+        for (int q = 1; q < Q; ++q) {
+          if (slot_of(q) < 0) continue;
+          const bool out_q = gone(q, yi);
+          if (EY[q] == 0) {
+            fc[q] = out_q ? own(OPP[q]) : pulled(q);
+          } else if (EY[q] > 0) {
+            if (out_q) fc[q] = own(OPP[q]);
+            fn[q] = pulled(q);
+          }
+        }
       }
     }
 #pragma unroll
-    for (int j = 0; j < K; ++j) {  // what planes yi and yi + 1 pull from plane yi
-#pragma unroll
-      for (int q = 1; q < Q; ++q) {
-        if (CIX[q] < 0) continue;
-        const bool out_q = gone(q, j, yi);
-        const float b = out_q ? own(OPP[q], j) : 0.0f;
-        if (EY[q] < 0) fc[j][q] = b;
-        else if (EY[q] == 0) fc[j][q] = out_q ? b : pulled(q, j);
-        else {
-          fc[j][q] = out_q ? b : fc[j][q];
-          fn[j][q] = pulled(q, j);
-        }
-      }
+    for (int q = 0; q < Q; ++q) {
+      if (EY[q] >= 0) fp[q] = fc[q];
+      if (EY[q] > 0) fc[q] = fn[q];
     }
-    __syncthreads();  // the next plane's first step overwrites LDS
-#pragma unroll
-    for (int j = 0; j < K; ++j)
-#pragma unroll
-      for (int q = 0; q < Q; ++q) {
-        fp[j][q] = fc[j][q];
-        if (EY[q] > 0) fc[j][q] = fn[j][q];
-      }
   }
 }
 
@@ -1406,24 +1442,20 @@ hipError_t launch_step(int storage, bool masked, bool sr, int block, int grid, h
   return step_mask<StF32, false>(masked, block, grid, st, d_lats, d_items, nitems, parity);
 }
 
-hipError_t launch_step2(int storage, hipStream_t st, const LatticeDev& L, int parity, int H) {
-  using G = step2::Geo<STEP2_TX, STEP2_TZ, STEP2_NT>;
-  // a workgroup's window (planes ya - 2 .. ya + H + 1) takes 32-bit byte offsets
-  if (H < 1 || storage != ST_F32 || ((unsigned long long)(H + 4) * L.nxz + 64) * Q * 4 >= (1ull << 32))
-    return hipErrorInvalidValue;
-  const int ntx = (L.nx + G::TX - 1) / G::TX, ntz = (L.nz + G::TZ - 1) / G::TZ, nch = (L.ny + H - 1) / H;
-  const dim3 grid((unsigned)(ntx * ntz * nch)), block(G::NT);
-  const bool runs = L.nx % 64 == 0;  // whole 64-node blocks per row
-  if (L.casetype == CASE_CHANNEL) {
+hipError_t launch_sweep(bool channel, bool runs, hipStream_t st, const LatticeDev* d_lats, const SweepItem* d_items,
+                        int nitems, int parity) {
+  if (nitems <= 0) return hipSuccess;
+  const dim3 grid((unsigned)nitems), block(SWEEP_NT);
+  if (channel) {
     if (runs)
-      hipLaunchKernelGGL((k_step2<StF32, G, true, true>), grid, block, 0, st, L, parity, H, ntx, ntz);
+      hipLaunchKernelGGL((k_sweep<StF32, true, true>), grid, block, 0, st, d_lats, d_items, parity);
     else
-      hipLaunchKernelGGL((k_step2<StF32, G, true, false>), grid, block, 0, st, L, parity, H, ntx, ntz);
+      hipLaunchKernelGGL((k_sweep<StF32, true, false>), grid, block, 0, st, d_lats, d_items, parity);
   } else {
     if (runs)
-      hipLaunchKernelGGL((k_step2<StF32, G, false, true>), grid, block, 0, st, L, parity, H, ntx, ntz);
+      hipLaunchKernelGGL((k_sweep<StF32, false, true>), grid, block, 0, st, d_lats, d_items, parity);
     else
-      hipLaunchKernelGGL((k_step2<StF32, G, false, false>), grid, block, 0, st, L, parity, H, ntx, ntz);
+      hipLaunchKernelGGL((k_sweep<StF32, false, false>), grid, block, 0, st, d_lats, d_items, parity);
   }
   return hipGetLastError();
 }

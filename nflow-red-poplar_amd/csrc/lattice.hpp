@@ -31,9 +31,6 @@ enum : int { SIDE_RHO = 0, SIDE_UIN = 1, SIDE_U0 = 4, SIDE_U1 = 8, SIDE_REC = 12
 // density is not a positive finite number and by the probe when some node's
 // rest population is not finite; cleared only by initialisation.
 enum : int { CTR_DIVERGED = 2, CTR_WORDS = 4 };
-// Two steps per launch (k_step2): x-z tiles of STEP2_TX x STEP2_TZ nodes,
-// STEP2_NT threads per workgroup (two nodes each).
-enum : int { STEP2_TX = 256, STEP2_TZ = 8, STEP2_NT = 1024 };
 
 // Exact unsigned division by a runtime constant d for n < 2^31:
 // floor(n / d) = (n * magic) >> shift with shift = 31 + ceil(log2 d) and
@@ -89,6 +86,17 @@ struct alignas(16) WorkItem {
   uint32_t pad;
 };
 
+// Work of one workgroup of k_sweep (two steps per launch): a tile of tx x tz
+// nodes of the x-z plane from (x0, z0), one per thread (tx tz <= SWEEP_NT, tz
+// <= SWEEP_ROWS), swept over the y planes [ya, ya + h); h = 0: no work.  The
+// exchange between the columns holds, per crossing population, SWEEP_SLOT0
+// elements where e_z = 0, at least tz (tx + 2), and SWEEP_SLOT1 where it is
+// not, at least (tz + 1) (tx + 2); two planes of it fill the LDS.
+enum : int { SWEEP_NT = 1024, SWEEP_ROWS = 32, SWEEP_SLOT0 = 1088, SWEEP_SLOT1 = 1296 };
+struct alignas(16) SweepItem {
+  int lat, x0, z0, ya, tx, tz, h, pad;
+};
+
 // Kernel launchers (kernels.hip).
 // masked: use the instantiation that honours LatticeDev::mask (any lattice of
 // the launch has solid nodes); sr: the one that can round stochastically (any
@@ -96,11 +104,13 @@ struct alignas(16) WorkItem {
 // nlat lattices.
 hipError_t launch_step(int storage, bool masked, bool sr, int block, int grid, hipStream_t st,
                        const LatticeDev* d_lats, int nlat, const WorkItem* d_items, int nitems, int parity);
-// Two steps in one launch (k_step2) for an FP32 cavity or channel lattice
-// without solid nodes: reads buf[parity ^ parity0] (and the side records of
-// that parity), writes the state two steps later to the other buffer (and
-// records); y planes are swept in chunks of H.
-hipError_t launch_step2(int storage, hipStream_t st, const LatticeDev& L, int parity, int H);
+// Two steps in one launch (k_sweep) for FP32 cavity and channel lattices
+// without solid nodes: every lattice of the work list reads buf[parity ^
+// parity0] (and the side records of that parity) and writes the state two
+// steps later to the other buffer (and records).  channel: some lattice is
+// one; runs: every nx is a multiple of 64.
+hipError_t launch_sweep(bool channel, bool runs, hipStream_t st, const LatticeDev* d_lats, const SweepItem* d_items,
+                        int nitems, int parity);
 // step0: the step count the initialised (or imported) state stands at; the
 // stochastic rounding of its look-ahead collision uses it.
 hipError_t launch_init(int storage, hipStream_t st, const LatticeDev& L, int cur, const float* src_aos, uint32_t step0);

@@ -265,6 +265,9 @@ int Server::tick() {
   if (k > 0)
     for (int w = 0; w < 2; ++w)
       if (!resident[w].empty()) {
+        // lattices come and go between ticks and some are read back: no tick
+        // ends with a two-step launch
+        batches[w].read_back = true;
         int rc = batches[w].run((int)k);
         if (rc) return rc;
       }

@@ -375,7 +375,7 @@ class Batch:
         return t.as_dict()
 
     def step2_height(self):
-        """y-chunk height of the two-step launches its runs use (0: one step per launch)."""
+        """y-chunk height its tuning names for two-step launches (see nflow_batch_step2_height)."""
         return _check(lib().nflow_batch_step2_height(self.h))
 
     def run(self, n):
