@@ -70,6 +70,9 @@ class Batch {
   bool sr_any = false;  // some lattice rounds its 16-bit stores stochastically
 
   int gparity = 0;  // parity argument of the next step launch
+  // step launches since the lattices' collision counters were last moved on:
+  // the count argument of the next one
+  uint32_t count = 0;
   hipGraphExec_t graph[2] = {nullptr, nullptr};
   int graph_steps_built = 0;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;

@@ -668,7 +668,7 @@ __device__ __forceinline__ void step_node(const LatticeDev& L, const WorkItem& w
 // element addressed is the same as with whole-array indexing.
 template <class St, int BS, bool MASK, bool SR>
 __global__ void __launch_bounds__(BS) NFLOW_STEP_ATTR k_step(const LatticeDev* __restrict__ lats, const WorkItem* __restrict__ items,
-                                             int nitems, int parity) {
+                                             int nitems, int parity, uint32_t count) {
   using T = typename St::T;
   for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
     const WorkItem wi = items[it];
@@ -676,13 +676,12 @@ __global__ void __launch_bounds__(BS) NFLOW_STEP_ATTR k_step(const LatticeDev* _
     const int p = parity ^ L.parity0;
     uint32_t sr_key = 0;
     if constexpr (SR) {
-      // this launch rounds with collision count ctr[p] (k_advance, launched
-      // after it, hands ctr[p] + 1 to the next launch in the other slot).
-      // Nothing in this kernel writes the counters, so the read goes through
+      // this launch rounds with collision count ctr[0] + count.
+      // Nothing in this kernel writes the counter, so the read goes through
       // the constant address space and becomes a scalar load: the step
       // kernel carries no store besides its populations and side records,
       // whose waits a store of its own would lengthen.
-      if (L.sr) sr_key = mix32(((__attribute__((address_space(4))) const uint32_t*)L.ctr)[p]);
+      if (L.sr) sr_key = mix32(*(__attribute__((address_space(4))) const uint32_t*)L.ctr + count);
     }
     if constexpr (NFLOW_AOSOA && NFLOW_BUFFER && St::buffer) {
       constexpr uint32_t B = 256 / sizeof(T);
@@ -703,16 +702,14 @@ __global__ void __launch_bounds__(BS) NFLOW_STEP_ATTR k_step(const LatticeDev* _
   }
 }
 
-// Collision counters of the stochastic rounding: after the launch that read
-// buf[p] (p = parity ^ parity0), ctr[p ^ 1] = ctr[p] + 1.
+// Collision counters of the stochastic rounding: ctr[0] += steps for every
+// lattice.  Step launches carry their distance from ctr[0] as an argument, so
+// this runs once per graph replay, whose arguments are fixed, and not after
+// every step: at 48^3 FP16 a second 3.6 us launch per step (7.25 -> 3.7 us).
 #if NFLOW_STORAGE_SET != 2  // the FP32 object carries it
-__global__ void __launch_bounds__(256) k_advance(const LatticeDev* __restrict__ lats, int nlat, int parity) {
+__global__ void __launch_bounds__(256) k_advance(const LatticeDev* __restrict__ lats, int nlat, uint32_t steps) {
   const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= nlat) return;
-  const LatticeDev& L = lats[i];
-  if (!L.sr) return;
-  const int p = parity ^ L.parity0;
-  L.ctr[p ^ 1] = L.ctr[p] + 1u;
+  if (i < nlat && lats[i].sr) lats[i].ctr[CTR_COUNT] += steps;
 }
 #endif
 
@@ -1025,15 +1022,19 @@ __global__ void __launch_bounds__(SWEEP_NT) k_sweep(const LatticeDev* __restrict
 // Initialisation (Initialize vertex, lbm_codelets.cpp:140-241) or import of
 // an arF array: the streamed state goes to buf[cur ^ 1] (what an export at
 // step 0 returns), its collision to buf[cur] (what the first step streams).
-// The state stands at step `step0`: its collision is rounded with that count
-// and the first step launch reads step0 + 1 from ctr[cur].
+// The state stands at step `step0`: its collision is rounded with that count;
+// count0 goes to ctr[0], for the first step launch to round with step0 + 1.
 template <class St>
-__global__ void __launch_bounds__(256) k_init(LatticeDev L, int cur, const float* __restrict__ src, uint32_t step0) {
+__global__ void __launch_bounds__(256) k_init(LatticeDev L, int cur, const float* __restrict__ src, uint32_t step0,
+                                              uint32_t count0) {
   using T = typename St::T;
   const uint32_t bn = blockIdx.x * 256u;  // the block's first node: buffers viewed from there
   const uint32_t n = bn + threadIdx.x, nr = threadIdx.x;
   if (n >= L.n) return;
-  if (n == 0) L.ctr[cur] = step0 + 1u;
+  if (n == 0) {
+    L.ctr[CTR_COUNT] = count0;
+    L.ctr[CTR_DIVERGED] = 0u;
+  }
   int x, y, z;
   coords(L, n, x, y, z);
   if (is_solid(L, n)) {
@@ -1328,19 +1329,23 @@ __global__ void __launch_bounds__(256) k_fma_chains(float* __restrict__ out, flo
 // ---------------------------------------------------------------------------
 template <class St, bool MASK, bool SR>
 static hipError_t step_bs(int block, int grid, hipStream_t st, const LatticeDev* d_lats, const WorkItem* d_items,
-                          int nitems, int parity) {
+                          int nitems, int parity, uint32_t count) {
   switch (block) {
     case 64:
-      hipLaunchKernelGGL((k_step<St, 64, MASK, SR>), dim3(grid), dim3(64), 0, st, d_lats, d_items, nitems, parity);
+      hipLaunchKernelGGL((k_step<St, 64, MASK, SR>), dim3(grid), dim3(64), 0, st, d_lats, d_items, nitems, parity,
+                         count);
       break;
     case 128:
-      hipLaunchKernelGGL((k_step<St, 128, MASK, SR>), dim3(grid), dim3(128), 0, st, d_lats, d_items, nitems, parity);
+      hipLaunchKernelGGL((k_step<St, 128, MASK, SR>), dim3(grid), dim3(128), 0, st, d_lats, d_items, nitems, parity,
+                         count);
       break;
     case 256:
-      hipLaunchKernelGGL((k_step<St, 256, MASK, SR>), dim3(grid), dim3(256), 0, st, d_lats, d_items, nitems, parity);
+      hipLaunchKernelGGL((k_step<St, 256, MASK, SR>), dim3(grid), dim3(256), 0, st, d_lats, d_items, nitems, parity,
+                         count);
       break;
     case 512:
-      hipLaunchKernelGGL((k_step<St, 512, MASK, SR>), dim3(grid), dim3(512), 0, st, d_lats, d_items, nitems, parity);
+      hipLaunchKernelGGL((k_step<St, 512, MASK, SR>), dim3(grid), dim3(512), 0, st, d_lats, d_items, nitems, parity,
+                         count);
       break;
     default: return hipErrorInvalidValue;
   }
@@ -1349,15 +1354,16 @@ static hipError_t step_bs(int block, int grid, hipStream_t st, const LatticeDev*
 
 template <class St, bool SR>
 static hipError_t step_mask(bool masked, int block, int grid, hipStream_t st, const LatticeDev* d_lats,
-                            const WorkItem* d_items, int nitems, int parity) {
-  return masked ? step_bs<St, true, SR>(block, grid, st, d_lats, d_items, nitems, parity)
-                : step_bs<St, false, SR>(block, grid, st, d_lats, d_items, nitems, parity);
+                            const WorkItem* d_items, int nitems, int parity, uint32_t count) {
+  return masked ? step_bs<St, true, SR>(block, grid, st, d_lats, d_items, nitems, parity, count)
+                : step_bs<St, false, SR>(block, grid, st, d_lats, d_items, nitems, parity, count);
 }
 
 // 16-bit storage (NFLOW_STORAGE_SET 2)
 hipError_t launch_step_h(int storage, bool masked, bool sr, int block, int grid, hipStream_t st,
-                         const LatticeDev* d_lats, const WorkItem* d_items, int nitems, int parity);
-hipError_t launch_init_h(int storage, hipStream_t st, const LatticeDev& L, int cur, const float* src, uint32_t step0);
+                         const LatticeDev* d_lats, const WorkItem* d_items, int nitems, int parity, uint32_t count);
+hipError_t launch_init_h(int storage, hipStream_t st, const LatticeDev& L, int cur, const float* src, uint32_t step0,
+                         uint32_t count0);
 hipError_t launch_export_h(int storage, hipStream_t st, const LatticeDev& L, int prev, int prev_streamed, float* aos,
                            float* rho, float* ux, float* uy, float* uz, double* partials, int grid);
 hipError_t launch_probe_h(int storage, hipStream_t st, const LatticeDev* d_lats, const WorkItem* d_items, int nitems,
@@ -1366,23 +1372,24 @@ hipError_t launch_probe_h(int storage, hipStream_t st, const LatticeDev* d_lats,
 #if NFLOW_STORAGE_SET == 2
 
 hipError_t launch_step_h(int storage, bool masked, bool sr, int block, int grid, hipStream_t st,
-                         const LatticeDev* d_lats, const WorkItem* d_items, int nitems, int parity) {
+                         const LatticeDev* d_lats, const WorkItem* d_items, int nitems, int parity, uint32_t count) {
   switch (storage) {
     case ST_F16:
-      return sr ? step_mask<StF16, true>(masked, block, grid, st, d_lats, d_items, nitems, parity)
-                : step_mask<StF16, false>(masked, block, grid, st, d_lats, d_items, nitems, parity);
+      return sr ? step_mask<StF16, true>(masked, block, grid, st, d_lats, d_items, nitems, parity, count)
+                : step_mask<StF16, false>(masked, block, grid, st, d_lats, d_items, nitems, parity, count);
     case ST_BF16:
-      return sr ? step_mask<StBF16, true>(masked, block, grid, st, d_lats, d_items, nitems, parity)
-                : step_mask<StBF16, false>(masked, block, grid, st, d_lats, d_items, nitems, parity);
+      return sr ? step_mask<StBF16, true>(masked, block, grid, st, d_lats, d_items, nitems, parity, count)
+                : step_mask<StBF16, false>(masked, block, grid, st, d_lats, d_items, nitems, parity, count);
   }
   return hipErrorInvalidValue;
 }
 
-hipError_t launch_init_h(int storage, hipStream_t st, const LatticeDev& L, int cur, const float* src, uint32_t step0) {
+hipError_t launch_init_h(int storage, hipStream_t st, const LatticeDev& L, int cur, const float* src, uint32_t step0,
+                         uint32_t count0) {
   const int grid = (int)((L.n + 255u) / 256u);
   switch (storage) {
-    case ST_F16: hipLaunchKernelGGL(k_init<StF16>, dim3(grid), dim3(256), 0, st, L, cur, src, step0); break;
-    case ST_BF16: hipLaunchKernelGGL(k_init<StBF16>, dim3(grid), dim3(256), 0, st, L, cur, src, step0); break;
+    case ST_F16: hipLaunchKernelGGL(k_init<StF16>, dim3(grid), dim3(256), 0, st, L, cur, src, step0, count0); break;
+    case ST_BF16: hipLaunchKernelGGL(k_init<StBF16>, dim3(grid), dim3(256), 0, st, L, cur, src, step0, count0); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -1431,15 +1438,17 @@ hipError_t launch_round16(hipStream_t st, int storage, const float* src, const u
 #else  // NFLOW_STORAGE_SET 1
 
 hipError_t launch_step(int storage, bool masked, bool sr, int block, int grid, hipStream_t st,
-                       const LatticeDev* d_lats, int nlat, const WorkItem* d_items, int nitems, int parity) {
+                       const LatticeDev* d_lats, const WorkItem* d_items, int nitems, int parity, uint32_t count) {
   if (grid <= 0 || nitems <= 0) return hipSuccess;
-  if (storage != ST_F32) {
-    const hipError_t e = launch_step_h(storage, masked, sr, block, grid, st, d_lats, d_items, nitems, parity);
-    if (e != hipSuccess || !sr) return e;
-    hipLaunchKernelGGL(k_advance, dim3((unsigned)((nlat + 255) / 256)), dim3(256), 0, st, d_lats, nlat, parity);
-    return hipGetLastError();
-  }
-  return step_mask<StF32, false>(masked, block, grid, st, d_lats, d_items, nitems, parity);
+  if (storage != ST_F32)
+    return launch_step_h(storage, masked, sr, block, grid, st, d_lats, d_items, nitems, parity, count);
+  return step_mask<StF32, false>(masked, block, grid, st, d_lats, d_items, nitems, parity, count);
+}
+
+hipError_t launch_advance(hipStream_t st, const LatticeDev* d_lats, int nlat, uint32_t steps) {
+  if (nlat <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_advance, dim3((unsigned)((nlat + 255) / 256)), dim3(256), 0, st, d_lats, nlat, steps);
+  return hipGetLastError();
 }
 
 hipError_t launch_sweep(bool channel, bool runs, hipStream_t st, const LatticeDev* d_lats, const SweepItem* d_items,
@@ -1460,10 +1469,11 @@ hipError_t launch_sweep(bool channel, bool runs, hipStream_t st, const LatticeDe
   return hipGetLastError();
 }
 
-hipError_t launch_init(int storage, hipStream_t st, const LatticeDev& L, int cur, const float* src, uint32_t step0) {
-  if (storage != ST_F32) return launch_init_h(storage, st, L, cur, src, step0);
+hipError_t launch_init(int storage, hipStream_t st, const LatticeDev& L, int cur, const float* src, uint32_t step0,
+                       uint32_t count0) {
+  if (storage != ST_F32) return launch_init_h(storage, st, L, cur, src, step0, count0);
   const int grid = (int)((L.n + 255u) / 256u);
-  hipLaunchKernelGGL(k_init<StF32>, dim3(grid), dim3(256), 0, st, L, cur, src, step0);
+  hipLaunchKernelGGL(k_init<StF32>, dim3(grid), dim3(256), 0, st, L, cur, src, step0, count0);
   return hipGetLastError();
 }
 

@@ -26,11 +26,11 @@ enum : int {
 // reads its inputs with one load and an outlet node with two.
 enum : int { SIDE_RHO = 0, SIDE_UIN = 1, SIDE_U0 = 4, SIDE_U1 = 8, SIDE_REC = 12 };
 
-// Words of LatticeDev::ctr: the two collision counters of the stochastic
-// rounding, then the divergence flag: set by the export when some node's
+// Words of LatticeDev::ctr: the collision counter of the stochastic rounding,
+// and the divergence flag: set by the export when some node's
 // density is not a positive finite number and by the probe when some node's
 // rest population is not finite; cleared only by initialisation.
-enum : int { CTR_DIVERGED = 2, CTR_WORDS = 4 };
+enum : int { CTR_COUNT = 0, CTR_DIVERGED = 2 };
 
 // Exact unsigned division by a runtime constant d for n < 2^31:
 // floor(n / d) = (n * magic) >> shift with shift = 31 + ceil(log2 d) and
@@ -63,9 +63,9 @@ struct alignas(16) LatticeDev {
   void* buf[2];
   float* side[2];
   const uint8_t* mask;  // solid nodes (non-zero), or null
-  // Collision counter of the stochastic rounding, ping-pong by parity like
-  // buf: the launch reading buf[p] rounds with ctr[p]; k_advance then writes
-  // ctr[p] + 1 to ctr[p ^ 1] (k_init writes the first value).
+  // Collision counter of the stochastic rounding (CTR_COUNT): a step launch
+  // rounds with it plus its own `count` argument; k_init writes the first
+  // value, k_advance moves it on.  And the divergence flag (CTR_DIVERGED).
   uint32_t* ctr;
   long long pstride;  // elements between population planes
   int nx, ny, nz, nxz;
@@ -100,10 +100,12 @@ struct alignas(16) SweepItem {
 // Kernel launchers (kernels.hip).
 // masked: use the instantiation that honours LatticeDev::mask (any lattice of
 // the launch has solid nodes); sr: the one that can round stochastically (any
-// lattice of the launch has LatticeDev::sr set), followed by k_advance over the
-// nlat lattices.
+// lattice of the launch has LatticeDev::sr set), with collision count ctr[0] +
+// count.
 hipError_t launch_step(int storage, bool masked, bool sr, int block, int grid, hipStream_t st,
-                       const LatticeDev* d_lats, int nlat, const WorkItem* d_items, int nitems, int parity);
+                       const LatticeDev* d_lats, const WorkItem* d_items, int nitems, int parity, uint32_t count);
+// ctr[0] += steps for every lattice that rounds stochastically
+hipError_t launch_advance(hipStream_t st, const LatticeDev* d_lats, int nlat, uint32_t steps);
 // Two steps in one launch (k_sweep) for FP32 cavity and channel lattices
 // without solid nodes: every lattice of the work list reads buf[parity ^
 // parity0] (and the side records of that parity) and writes the state two
@@ -112,8 +114,10 @@ hipError_t launch_step(int storage, bool masked, bool sr, int block, int grid, h
 hipError_t launch_sweep(bool channel, bool runs, hipStream_t st, const LatticeDev* d_lats, const SweepItem* d_items,
                         int nitems, int parity);
 // step0: the step count the initialised (or imported) state stands at; the
-// stochastic rounding of its look-ahead collision uses it.
-hipError_t launch_init(int storage, hipStream_t st, const LatticeDev& L, int cur, const float* src_aos, uint32_t step0);
+// stochastic rounding of its look-ahead collision uses it.  count0: the first
+// value of ctr[0].
+hipError_t launch_init(int storage, hipStream_t st, const LatticeDev& L, int cur, const float* src_aos, uint32_t step0,
+                       uint32_t count0);
 hipError_t launch_export(int storage, hipStream_t st, const LatticeDev& L, int prev, int prev_streamed, float* aos,
                          float* rho, float* ux, float* uy, float* uz, double* partials, int* nblocks_out);
 hipError_t launch_reduce(hipStream_t st, const double* partials, int nblocks, double* out5);

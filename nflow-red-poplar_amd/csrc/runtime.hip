@@ -363,9 +363,9 @@ int Batch::upload_tables() {
 
 int Batch::init_lattice(int idx, const float* d_src, long long step0) {
   HostLattice& h = lats[idx];
-  // counters and divergence flag start afresh (k_init sets the counter)
-  NFLOW_HIP(hipMemsetAsync(h.dev.ctr, 0, CTR_WORDS * sizeof(uint32_t), stream));
-  NFLOW_HIP(launch_init(storage, stream, h.dev, gparity, d_src, (uint32_t)step0));
+  // k_init also starts the counter (the next launch rounds with ctr[0] + count)
+  // and the divergence flag afresh
+  NFLOW_HIP(launch_init(storage, stream, h.dev, gparity, d_src, (uint32_t)step0, (uint32_t)step0 + 1u - count));
   h.cur = gparity;
   h.steps_done = step0;
   h.prev_streamed = true;
@@ -388,9 +388,11 @@ int Batch::build_graph(int parity) {
   int p = parity;
   hipError_t err = hipSuccess;
   for (int s = 0; s < tuning.graph_steps && err == hipSuccess; ++s) {
-    err = launch_step(storage, masked, sr_any, tuning.block, grid, stream, d_lats, (int)lats.size(), d_items, nitems, p);
+    err = launch_step(storage, masked, sr_any, tuning.block, grid, stream, d_lats, d_items, nitems, p, (uint32_t)s);
     p ^= 1;
   }
+  if (sr_any && err == hipSuccess)
+    err = launch_advance(stream, d_lats, (int)lats.size(), (uint32_t)tuning.graph_steps);
   hipError_t e2 = hipStreamEndCapture(stream, &g);
   if (err != hipSuccess || e2 != hipSuccess) {
     if (g) (void)hipGraphDestroy(g);
@@ -437,12 +439,16 @@ int Batch::launch_steps(int nsteps) {
       if (rc) return rc;
     }
     const int reps = left / gs;
+    // a replay's launches count from 0
+    if (sr_any && count) NFLOW_HIP(launch_advance(stream, d_lats, (int)lats.size(), count));
+    count = 0;
     for (int r = 0; r < reps; ++r) NFLOW_HIP(hipGraphLaunch(graph[gparity], stream));
     left -= reps * gs;
     launches += (long long)reps * gs;
   }
   for (int s = 0; s < left; ++s) {
-    NFLOW_HIP(launch_step(storage, masked, sr_any, tuning.block, grid, stream, d_lats, (int)lats.size(), d_items, nitems, gparity));
+    NFLOW_HIP(launch_step(storage, masked, sr_any, tuning.block, grid, stream, d_lats, d_items, nitems, gparity, count));
+    if (sr_any) ++count;
     gparity ^= 1;
     ++launches;
   }
@@ -467,9 +473,9 @@ int Batch::settle_pair() {
   // every change of the lattice set or the tuning settles first, so the
   // lattices and tables are those of that launch
   if (tables_dirty || !all) return fail(NFLOW_ESTATE, "settle_pair: tables changed after a two-step launch");
-  const int p = gparity ^ 1, n = (int)lats.size();  // p: the parity the pair was launched with
-  NFLOW_HIP(launch_step(storage, masked, sr_any, tuning.block, grid, stream, d_lats, n, d_items, nitems, p));
-  NFLOW_HIP(launch_step(storage, masked, sr_any, tuning.block, grid, stream, d_lats, n, d_items, nitems, p ^ 1));
+  const int p = gparity ^ 1;  // the parity the pair was launched with
+  NFLOW_HIP(launch_step(storage, masked, sr_any, tuning.block, grid, stream, d_lats, d_items, nitems, p, 0u));
+  NFLOW_HIP(launch_step(storage, masked, sr_any, tuning.block, grid, stream, d_lats, d_items, nitems, p ^ 1, 0u));
   launches += 2;
   gparity = p;
   for (auto& h : lats) {
