@@ -4,6 +4,7 @@
 #include <cstddef>
 #include <vector>
 
+#include "hostcopy.hpp"
 #include "lattice.hpp"
 #include "nflow.h"
 
@@ -95,6 +96,7 @@ class Batch {
   uint32_t* d_flags = nullptr;  // divergence flags of every lattice, gathered
   size_t d_flags_cap = 0;
   std::vector<uint32_t> h_flags;
+  HostCopy host;  // copies to and from the callers' arrays
 
   Batch() = default;
   Batch(const Batch&) = delete;

@@ -1190,9 +1190,11 @@ __global__ void __launch_bounds__(EXPORT_BS) k_export(LatticeDev L, int prev, in
 }
 
 #if NFLOW_STORAGE_SET != 2  // the FP32 object carries it
+// out[0..4]: the sums; out[5]: 1 when the lattice is marked as diverged, else 0.
 __global__ void __launch_bounds__(256) k_reduce(const double* __restrict__ partials, int nblocks,
-                                                double* __restrict__ out) {
+                                                const uint32_t* __restrict__ ctr, double* __restrict__ out) {
   __shared__ double sh[256];
+  if (threadIdx.x == 0) out[5] = ctr[CTR_DIVERGED] ? 1.0 : 0.0;
   for (int c = 0; c < 5; ++c) {
     double v = 0.0;
     for (int i = threadIdx.x; i < nblocks; i += 256) v += partials[(size_t)i * 5 + c];
@@ -1490,8 +1492,8 @@ hipError_t launch_export(int storage, hipStream_t st, const LatticeDev& L, int p
   return hipGetLastError();
 }
 
-hipError_t launch_reduce(hipStream_t st, const double* partials, int nblocks, double* out5) {
-  hipLaunchKernelGGL(k_reduce, dim3(1), dim3(256), 0, st, partials, nblocks, out5);
+hipError_t launch_reduce(hipStream_t st, const double* partials, int nblocks, const uint32_t* ctr, double* out6) {
+  hipLaunchKernelGGL(k_reduce, dim3(1), dim3(256), 0, st, partials, nblocks, ctr, out6);
   return hipGetLastError();
 }
 

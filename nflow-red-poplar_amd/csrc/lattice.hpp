@@ -120,7 +120,9 @@ hipError_t launch_init(int storage, hipStream_t st, const LatticeDev& L, int cur
                        uint32_t count0);
 hipError_t launch_export(int storage, hipStream_t st, const LatticeDev& L, int prev, int prev_streamed, float* aos,
                          float* rho, float* ux, float* uy, float* uz, double* partials, int* nblocks_out);
-hipError_t launch_reduce(hipStream_t st, const double* partials, int nblocks, double* out5);
+// out6: the five sums of the export's partials, then 1 or 0 for the divergence
+// flag at ctr
+hipError_t launch_reduce(hipStream_t st, const double* partials, int nblocks, const uint32_t* ctr, double* out6);
 // rest-population probe of every node of a work list (items of at most 512
 // nodes), newest state = the buffer the launch with `parity` would read
 hipError_t launch_probe(int storage, hipStream_t st, const LatticeDev* d_lats, const WorkItem* d_items, int nitems,

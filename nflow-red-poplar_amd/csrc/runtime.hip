@@ -144,8 +144,8 @@ int lattice_upload_inlet(HostLattice& h, hipStream_t st) {
       const double xi = 2.0 * ((double)(splitmix64(key) >> 11) * (1.0 / 9007199254740992.0)) - 1.0;
       u = (float)(in.inlet_peak * 16.0 * eta * (1.0 - eta) * zeta * (1.0 - zeta) * (1.0 + in.perturb * xi));
     }
-  for (int b = 0; b < 2; ++b)
-    NFLOW_HIP(hipMemcpyAsync(h.dev.side[b], rec.data(), rec.size() * sizeof(float), hipMemcpyHostToDevice, st));
+  NFLOW_HIP(hipMemcpyAsync(h.dev.side[0], rec.data(), rec.size() * sizeof(float), hipMemcpyHostToDevice, st));
+  NFLOW_HIP(hipMemcpyAsync(h.dev.side[1], h.dev.side[0], rec.size() * sizeof(float), hipMemcpyDeviceToDevice, st));
   std::vector<uint8_t> m;
   if (in.casetype == NFLOW_PIPE) {  // keSetNodeType, kernel.cu:1078-1094
     m.resize((size_t)h.dev.n);
@@ -601,21 +601,25 @@ int Batch::export_one(int idx, float* aos, float* rho, float* ux, float* uy, flo
   float* m = rho ? macro : nullptr;
   NFLOW_HIP(launch_export(storage, stream, h.dev, prev, prev_streamed, aos ? d_aos : nullptr, m, m ? m + n : nullptr,
                           m ? m + 2 * n : nullptr, m ? m + 3 * n : nullptr, diag5 ? partials : nullptr, &nblocks));
-  if (diag5) NFLOW_HIP(launch_reduce(stream, partials, nblocks, out5));
-  if (aos) NFLOW_HIP(hipMemcpyAsync(aos, d_aos, padded_count(h.in) * sizeof(float), hipMemcpyDeviceToHost, stream));
-  if (rho) {
-    NFLOW_HIP(hipMemcpyAsync(rho, m, n * sizeof(float), hipMemcpyDeviceToHost, stream));
-    NFLOW_HIP(hipMemcpyAsync(ux, m + n, n * sizeof(float), hipMemcpyDeviceToHost, stream));
-    NFLOW_HIP(hipMemcpyAsync(uy, m + 2 * n, n * sizeof(float), hipMemcpyDeviceToHost, stream));
-    NFLOW_HIP(hipMemcpyAsync(uz, m + 3 * n, n * sizeof(float), hipMemcpyDeviceToHost, stream));
+  if (diag5) NFLOW_HIP(launch_reduce(stream, partials, nblocks, h.dev.ctr, out5));
+  int rc = 0;
+  if (aos) {
+    void* to[1] = {aos};
+    rc = host.to_host(stream, d_aos, padded_count(h.in) * sizeof(float), to, 1);
   }
-  if (diag5) NFLOW_HIP(hipMemcpyAsync(diag5, out5, 5 * sizeof(double), hipMemcpyDeviceToHost, stream));
-  uint32_t flag = 0;
-  if (diverged)
-    NFLOW_HIP(hipMemcpyAsync(&flag, h.dev.ctr + CTR_DIVERGED, sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
-  NFLOW_HIP(hipStreamSynchronize(stream));
-  if (diverged) *diverged = flag ? 1 : 0;
-  return 0;
+  if (rho && !rc) {  // rho, ux, uy, uz lie one after another
+    void* to[4] = {rho, ux, uy, uz};
+    rc = host.to_host(stream, m, n * sizeof(float), to, 4);
+  }
+  if (diag5 && !rc) {  // the five sums and the divergence flag
+    double d[6];
+    void* to[1] = {d};
+    rc = host.to_host(stream, out5, sizeof(d), to, 1);
+    std::copy(d, d + 5, diag5);
+    if (diverged) *diverged = d[5] != 0.0 ? 1 : 0;
+  }
+  if (!rc) NFLOW_HIP(hipStreamSynchronize(stream));
+  return rc;
 }
 
 int Batch::import_one(int idx, const float* aos_host, long long step0) {
@@ -623,7 +627,8 @@ int Batch::import_one(int idx, const float* aos_host, long long step0) {
   HostLattice& h = lats[idx];
   int rc = ensure_scratch(padded_count(h.in), 0, 0, 0);
   if (rc) return rc;
-  NFLOW_HIP(hipMemcpyAsync(d_aos, aos_host, padded_count(h.in) * sizeof(float), hipMemcpyHostToDevice, stream));
+  rc = host.to_device(stream, d_aos, aos_host, padded_count(h.in) * sizeof(float));
+  if (rc) return rc;
   rc = init_lattice(idx, d_aos, step0);
   if (rc) return rc;
   NFLOW_HIP(hipStreamSynchronize(stream));
@@ -1150,11 +1155,9 @@ extern "C" int nflow_diagnostics_noalloc(nflow_solver* s, double* mass, double m
   int nblocks = 0;
   NFLOW_HIP(launch_export(b.storage, b.stream, h.dev, h.cur ^ 1, h.prev_streamed ? 1 : 0, nullptr, nullptr, nullptr,
                           nullptr, nullptr, partials, &nblocks));
-  NFLOW_HIP(launch_reduce(b.stream, partials, nblocks, sums));
-  double d[5];
-  uint32_t flag = 0;
+  NFLOW_HIP(launch_reduce(b.stream, partials, nblocks, h.dev.ctr, sums));
+  double d[6];
   NFLOW_HIP(hipMemcpyAsync(d, sums, sizeof(d), hipMemcpyDeviceToHost, b.stream));
-  NFLOW_HIP(hipMemcpyAsync(&flag, h.dev.ctr + CTR_DIVERGED, sizeof(flag), hipMemcpyDeviceToHost, b.stream));
   NFLOW_HIP(hipStreamSynchronize(b.stream));
   *mass = d[0];
   mom[0] = d[1];
@@ -1163,7 +1166,7 @@ extern "C" int nflow_diagnostics_noalloc(nflow_solver* s, double* mass, double m
   *drho_l1 = d[4];
   bool finite = true;
   for (double v : d) finite = finite && std::isfinite(v);
-  if (flag || !finite)
+  if (d[5] != 0.0 || !finite)
     return fail(NFLOW_EDIVERGED, "lattice diverged: a node's density was not a positive finite number (mass %g)", d[0]);
   return 0;
 }

@@ -18,17 +18,20 @@
 // requests whose relaxation time lies below it are kept in FP32 storage: they
 // form a second batch, stepped in its own launch on its own stream each tick.
 #include <hip/hip_runtime.h>
+#include <sys/mman.h>
 
 #include <algorithm>
 #include <cmath>
 #include <atomic>
 #include <chrono>
 #include <condition_variable>
+#include <cstdlib>
 #include <cstring>
 #include <deque>
 #include <map>
 #include <mutex>
 #include <thread>
+#include <utility>
 #include <vector>
 
 #include "batch.hpp"
@@ -93,6 +96,33 @@ class Arena {
   std::map<size_t, size_t> free_;  // offset -> length
 };
 
+// rho, ux, uy, uz of a finished request, n floats each.  Fresh memory, not
+// cleared, in huge pages where it is large: clearing it first and faulting it
+// in 4 KiB pages took longer than the copy from the device.
+class Fields {
+ public:
+  Fields() = default;
+  explicit Fields(size_t n) : n_(n) {
+    const size_t bytes = 4 * n * sizeof(float), align = size_t(2) << 20, all = (bytes + align - 1) / align * align;
+    p_ = static_cast<float*>(bytes < align ? std::malloc(bytes) : std::aligned_alloc(align, all));
+    if (p_ && bytes >= align) (void)madvise(p_, all, MADV_HUGEPAGE);
+  }
+  Fields(Fields&& o) noexcept : p_(std::exchange(o.p_, nullptr)), n_(o.n_) {}
+  Fields& operator=(Fields&& o) noexcept {
+    std::swap(p_, o.p_);
+    std::swap(n_, o.n_);
+    return *this;
+  }
+  ~Fields() { std::free(p_); }
+  float* at(int k) const { return p_ + k * n_; }
+  size_t n() const { return n_; }
+  explicit operator bool() const { return p_ != nullptr; }
+
+ private:
+  float* p_ = nullptr;
+  size_t n_ = 0;
+};
+
 struct Pending {
   nflow_request req;
   double submit_s;
@@ -121,7 +151,7 @@ class Server {
   std::deque<Pending> queue;    // submitted, not yet seen by the worker (under mu)
   std::deque<Pending> waiting;  // seen by the worker, not admitted (worker only)
   std::deque<nflow_result> results;
-  std::map<unsigned long long, std::vector<float>> fields;
+  std::map<unsigned long long, Fields> fields;
   std::vector<Resident> resident[2];  // parallel to batches[w].lats
   nflow_server_stats st{};
   bool stop = false;
@@ -217,15 +247,14 @@ void Server::finish(int w, size_t i, bool diverged) {
   res.submit_s = r.submit_s;
   res.admit_s = r.admit_s;
   double d[5] = {0, 0, 0, 0, 0};
-  std::vector<float> f;
+  Fields f;
   int rc;
   // the lattice leaves: the export works inside its own (idle) population
   // buffer, so finishing allocates no device memory outside the arena
   if (r.req.want_fields && !diverged) {
-    const size_t n = h.dev.n;
-    f.resize(4 * n);
-    rc = batch.export_one((int)i, nullptr, f.data(), f.data() + n, f.data() + 2 * n, f.data() + 3 * n, d, nullptr,
-                          true);
+    f = Fields(h.dev.n);
+    rc = f ? batch.export_one((int)i, nullptr, f.at(0), f.at(1), f.at(2), f.at(3), d, nullptr, true)
+           : fail(NFLOW_ENOMEM, "fields of a finished request");
   } else {
     rc = batch.export_one((int)i, nullptr, nullptr, nullptr, nullptr, nullptr, d, nullptr, true);
   }
@@ -438,15 +467,16 @@ extern "C" int nflow_server_fetch_macro(nflow_server* sv, unsigned long long tag
                                         float* uz) {
   if (!sv || !rho || !ux || !uy || !uz) return fail(NFLOW_EINVAL, "nflow_server_fetch_macro: null argument");
   Server& s = sv->s;
-  std::lock_guard<std::mutex> lk(s.mu);
-  auto it = s.fields.find(tag);
-  if (it == s.fields.end()) return fail(NFLOW_ENOTFOUND, "no fields kept for tag %llu", tag);
-  const size_t n = it->second.size() / 4;
-  std::memcpy(rho, it->second.data(), n * sizeof(float));
-  std::memcpy(ux, it->second.data() + n, n * sizeof(float));
-  std::memcpy(uy, it->second.data() + 2 * n, n * sizeof(float));
-  std::memcpy(uz, it->second.data() + 3 * n, n * sizeof(float));
-  s.fields.erase(it);
+  Fields f;
+  {
+    std::lock_guard<std::mutex> lk(s.mu);
+    auto it = s.fields.find(tag);
+    if (it == s.fields.end()) return fail(NFLOW_ENOTFOUND, "no fields kept for tag %llu", tag);
+    f = std::move(it->second);
+    s.fields.erase(it);
+  }
+  float* const to[4] = {rho, ux, uy, uz};
+  for (int k = 0; k < 4; ++k) parallel_memcpy(to[k], f.at(k), f.n() * sizeof(float));
   return 0;
 }
 
