@@ -16,9 +16,11 @@
 #include <cstddef>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <new>
 #include <system_error>
 #include <thread>
+#include <utility>
 
 #include "errors.hpp"
 #include "nflow.h"
@@ -40,9 +42,13 @@ void run_threads(int extra, F f, Main mine) {
   for (int i = 0; i < n; ++i) t[i].join();
 }
 
+// Helpers for a copy; 0: too small for threads.  From 3 MiB eight of them
+// halve the time into fresh pages (8 MiB 1.9 -> 0.9 ms), and lose little where
+// malloc hands the same pages out again (0.5 -> 0.7 ms).  1.7 MiB is 130 us as
+// the runtime's own pageable copies, 310 us through the chunks.
 inline int copy_threads(size_t bytes) {
   const unsigned hw = std::thread::hardware_concurrency();
-  return (int)std::min<size_t>({bytes >> 20, 8, hw ? hw : 1});
+  return bytes < (3u << 20) ? 0 : (int)std::min<size_t>({bytes >> 19, 8, hw ? hw : 1});
 }
 
 // memcpy by several threads (fresh destination pages are faulted in by all)
@@ -53,33 +59,93 @@ inline void parallel_memcpy(void* dst, const void* src, size_t n) {
     for (size_t o; (o = next.fetch_add(PIECE)) < n;)
       std::memcpy(static_cast<char*>(dst) + o, static_cast<const char*>(src) + o, std::min(PIECE, n - o));
   };
-  run_threads(copy_threads(n) - 1, work, [&](int) { work(); });
+  run_threads(copy_threads(n), work, [&](int) { work(); });
 }
 
-// The pinned chunks of one batch: used by one host thread at a time, on the
-// batch's stream.  16 MiB, taken at the first copy and held as the export
-// scratch on the device is.
+// Pinned chunks and the events of the copies through them.
+struct Pinned {
+  static constexpr size_t CHUNK = 2u << 20, SLOTS = 8;
+  char* buf = nullptr;
+  int device = -1;  // the events' device
+  hipEvent_t ev[SLOTS] = {};
+  Pinned() = default;
+  Pinned(const Pinned&) = delete;
+  Pinned& operator=(const Pinned&) = delete;
+  ~Pinned() {
+    for (auto& e : ev)
+      if (e) (void)hipEventDestroy(e);
+    if (buf) (void)hipHostFree(buf);
+  }
+  bool open(int dev) {
+    device = dev;
+    bool ok = true;
+    for (auto& e : ev) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+    void* p = nullptr;
+    ok = ok && hipHostMalloc(&p, SLOTS * CHUNK, hipHostMallocPortable) == hipSuccess;
+    if (!ok) (void)hipGetLastError();
+    buf = ok ? static_cast<char*>(p) : nullptr;
+    return ok;
+  }
+};
+
+// The idle Pinned of the process, two at most, kept while any HostCopy lives
+// and given back with the last: a new solver's first read-back finds them
+// ready (allocating 16 MiB of pinned memory takes 1 to 2 ms).  Copies that
+// overlap each hold one of their own.
+class PinnedPool {
+ public:
+  static std::shared_ptr<PinnedPool> get() {
+    static std::mutex mu;
+    static std::weak_ptr<PinnedPool> pool;
+    std::lock_guard<std::mutex> lk(mu);
+    std::shared_ptr<PinnedPool> p = pool.lock();
+    if (!p) pool = p = std::make_shared<PinnedPool>();
+    return p;
+  }
+  std::unique_ptr<Pinned> take(int device) {
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      for (auto& p : idle_)
+        if (p && p->device == device) return std::move(p);
+    }
+    std::unique_ptr<Pinned> p(new (std::nothrow) Pinned);
+    if (p && !p->open(device)) p.reset();
+    return p;
+  }
+  void give(std::unique_ptr<Pinned> p) {
+    std::lock_guard<std::mutex> lk(mu_);
+    for (auto& q : idle_)
+      if (!q) {
+        q = std::move(p);
+        return;
+      }
+  }
+
+ private:
+  std::mutex mu_;
+  std::unique_ptr<Pinned> idle_[2];
+};
+
+// One batch's copies: one host thread at a time, on the batch's stream and
+// device.
 class HostCopy {
  public:
-  HostCopy() = default;
-  HostCopy(const HostCopy&) = delete;
-  HostCopy& operator=(const HostCopy&) = delete;
-  ~HostCopy() {
-    for (auto& e : ev_)
-      if (e) (void)hipEventDestroy(e);
-    if (buf_) (void)hipHostFree(buf_);
-  }
+  int device = 0;
 
   // `parts` consecutive ranges of n bytes from src on the device to dst[0],
   // dst[1], ...; complete on return, and so is all earlier work of the stream.
   int to_host(hipStream_t st, const void* src, size_t n, void* const* dst, int parts) {
     const size_t total = n * parts;
-    if (!open()) {  // no pinned memory: plain copies
+    const int helpers = copy_threads(total);
+    const Lease lease(*this, helpers > 0 || total <= SMALL);
+    if (!lease) {  // plain copies
       for (int i = 0; i < parts; ++i)
         NFLOW_HIP(hipMemcpyAsync(dst[i], static_cast<const char*>(src) + i * n, n, hipMemcpyDeviceToHost, st));
       NFLOW_HIP(hipStreamSynchronize(st));
       return 0;
     }
+    char* const buf = lease->buf;
+    hipEvent_t* const ev = lease->ev;
     auto put = [&](size_t off, const char* from, size_t len) {  // [off, off + len) of the total
       while (len) {
         const size_t i = off / n, o = off % n, l = std::min(len, n - o);
@@ -89,59 +155,66 @@ class HostCopy {
         len -= l;
       }
     };
-    if (total <= PIECE) {
-      NFLOW_HIP(hipMemcpyAsync(buf_, src, total, hipMemcpyDeviceToHost, st));
+    if (helpers == 0) {  // one short copy on the link (0.5 MiB: 69 us, as four plain ones 278 us)
+      NFLOW_HIP(hipMemcpyAsync(buf, src, total, hipMemcpyDeviceToHost, st));
       NFLOW_HIP(hipStreamSynchronize(st));
-      put(0, buf_, total);
+      put(0, buf, total);
       return 0;
     }
-    const size_t pieces = (total + PIECE - 1) / PIECE;
+    const size_t pieces = (total + PIECE - 1) / PIECE, chunks = (total + CHUNK - 1) / CHUNK;
     std::atomic<size_t> ready{0}, next{0};  // chunks on the host; next piece to move on
     std::atomic<size_t> moved[SLOTS];       // pieces moved out of each slot, over the whole copy
     for (auto& m : moved) m.store(0);
     std::atomic<bool> stop{false};
+    auto move_on = [&](size_t i) {
+      const size_t c = i / PER, off = i * PIECE;
+      put(off, buf + (c % SLOTS) * CHUNK + (off - c * CHUNK), std::min(PIECE, total - off));
+      moved[c % SLOTS].fetch_add(1, std::memory_order_release);
+    };
     auto work = [&] {
       for (size_t i; !stop.load() && (i = next.fetch_add(1)) < pieces;) {
-        const size_t c = i / PER, off = i * PIECE;
-        while (ready.load(std::memory_order_acquire) <= c) {
+        while (ready.load(std::memory_order_acquire) <= i / PER) {
           if (stop.load()) return;
           std::this_thread::yield();
         }
-        put(off, buf_ + (c % SLOTS) * CHUNK + (off - c * CHUNK), std::min(PIECE, total - off));
-        moved[c % SLOTS].fetch_add(1, std::memory_order_release);
+        move_on(i);
       }
     };
     hipError_t err = hipSuccess;
-    run_threads(copy_threads(total), work, [&](int helpers) {
-      const size_t chunks = (total + CHUNK - 1) / CHUNK;
-      size_t issued = 0, done = 0;
-      auto slot_free = [&](size_t c) {  // every earlier chunk of the slot moved on?
-        return c < SLOTS || moved[c % SLOTS].load(std::memory_order_acquire) >= (c / SLOTS) * PER;
-      };
+    size_t issued = 0, done = 0;
+    auto issue = [&] {  // keep half of the slots on the link, where they are free
+      while (issued < chunks && issued < done + SLOTS / 2 && err == hipSuccess &&
+             (issued < SLOTS || moved[issued % SLOTS].load(std::memory_order_acquire) >= (issued / SLOTS) * PER)) {
+        const size_t off = issued * CHUNK;
+        err = hipMemcpyAsync(buf + (issued % SLOTS) * CHUNK, static_cast<const char*>(src) + off,
+                             std::min(CHUNK, total - off), hipMemcpyDeviceToHost, st);
+        if (err == hipSuccess) err = hipEventRecord(ev[issued % SLOTS], st);
+        ++issued;
+      }
+    };
+    issue();
+    run_threads(err == hipSuccess ? helpers : 0, work, [&](int running) {
       while (done < chunks && err == hipSuccess) {
-        while (issued < chunks && issued < done + SLOTS / 2 && slot_free(issued) && err == hipSuccess) {
-          const size_t off = issued * CHUNK;
-          err = hipMemcpyAsync(buf_ + (issued % SLOTS) * CHUNK, static_cast<const char*>(src) + off,
-                               std::min(CHUNK, total - off), hipMemcpyDeviceToHost, st);
-          if (err == hipSuccess) err = hipEventRecord(ev_[issued % SLOTS], st);
-          ++issued;
-        }
+        issue();
         if (err == hipSuccess && done < issued) {
-          err = hipEventSynchronize(ev_[done % SLOTS]);
-          if (err == hipSuccess) ready.store(++done, std::memory_order_release);
-          if (helpers == 0 && err == hipSuccess)  // alone: move it on before the next
-            for (size_t i; (i = next.load()) < std::min(done * PER, pieces);) {
+          err = hipEventSynchronize(ev[done % SLOTS]);
+          if (err != hipSuccess) break;
+          ready.store(++done, std::memory_order_release);
+          if (running == 0) {  // alone: move it on, with the next ones on the link
+            issue();
+            for (size_t i = next.load(); i < std::min(done * PER, pieces); ++i) {
               next.store(i + 1);
-              const size_t c = i / PER, off = i * PIECE;
-              put(off, buf_ + (c % SLOTS) * CHUNK + (off - c * CHUNK), std::min(PIECE, total - off));
-              moved[c % SLOTS].fetch_add(1, std::memory_order_release);
+              move_on(i);
             }
+          }
         } else if (err == hipSuccess) {
           std::this_thread::yield();
         }
       }
-      if (err != hipSuccess) stop.store(true);
-      else work();  // lend a hand with what is left
+      if (err != hipSuccess)
+        stop.store(true);
+      else
+        work();  // lend a hand with what is left
     });
     if (err != hipSuccess) {
       (void)hipStreamSynchronize(st);
@@ -153,11 +226,14 @@ class HostCopy {
   // n bytes from the host to dst on the device, in stream order; src may be
   // reused on return (the last chunks may still be on their way).
   int to_device(hipStream_t st, void* dst, const void* src, size_t n) {
-    if (n <= CHUNK || !open()) {
+    const Lease lease(*this, copy_threads(n) > 0);
+    if (!lease) {
       NFLOW_HIP(hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, st));
       NFLOW_HIP(hipStreamSynchronize(st));
       return 0;
     }
+    char* const buf = lease->buf;
+    hipEvent_t* const ev = lease->ev;
     const size_t pieces = (n + PIECE - 1) / PIECE, chunks = (n + CHUNK - 1) / CHUNK;
     std::atomic<size_t> freed{0}, next{0};  // chunks that have left their slots; next piece to bring
     std::atomic<size_t> filled[SLOTS];      // pieces brought into each slot, over the whole copy
@@ -165,7 +241,7 @@ class HostCopy {
     std::atomic<bool> stop{false};
     auto bring = [&](size_t i) {
       const size_t c = i / PER, off = i * PIECE;
-      std::memcpy(buf_ + (c % SLOTS) * CHUNK + (off - c * CHUNK), static_cast<const char*>(src) + off,
+      std::memcpy(buf + (c % SLOTS) * CHUNK + (off - c * CHUNK), static_cast<const char*>(src) + off,
                   std::min(PIECE, n - off));
       filled[c % SLOTS].fetch_add(1, std::memory_order_release);
     };
@@ -183,7 +259,7 @@ class HostCopy {
       for (size_t c = 0; c < chunks && err == hipSuccess; ++c) {
         // chunk c - SLOTS / 2 has left: its slot may be filled again
         if (c >= SLOTS / 2) {
-          err = hipEventSynchronize(ev_[(c - SLOTS / 2) % SLOTS]);
+          err = hipEventSynchronize(ev[(c - SLOTS / 2) % SLOTS]);
           if (err != hipSuccess) break;
           freed.store(c - SLOTS / 2 + 1, std::memory_order_release);
         }
@@ -194,9 +270,9 @@ class HostCopy {
           }
         const size_t mine = std::min<size_t>(PER, pieces - c * PER);
         while (filled[c % SLOTS].load(std::memory_order_acquire) < (c / SLOTS) * PER + mine) std::this_thread::yield();
-        err = hipMemcpyAsync(static_cast<char*>(dst) + c * CHUNK, buf_ + (c % SLOTS) * CHUNK,
+        err = hipMemcpyAsync(static_cast<char*>(dst) + c * CHUNK, buf + (c % SLOTS) * CHUNK,
                              std::min(CHUNK, n - c * CHUNK), hipMemcpyHostToDevice, st);
-        if (err == hipSuccess) err = hipEventRecord(ev_[c % SLOTS], st);
+        if (err == hipSuccess) err = hipEventRecord(ev[c % SLOTS], st);
       }
       if (err != hipSuccess) stop.store(true);
     });
@@ -207,26 +283,22 @@ class HostCopy {
   }
 
  private:
-  static constexpr size_t CHUNK = 2u << 20, SLOTS = 8, PIECE = 256u << 10, PER = CHUNK / PIECE;
-  char* buf_ = nullptr;
-  hipEvent_t ev_[SLOTS] = {};
-  bool failed_ = false;
+  static constexpr size_t CHUNK = Pinned::CHUNK, SLOTS = Pinned::SLOTS, PIECE = 256u << 10, PER = CHUNK / PIECE,
+                          SMALL = 1u << 20;
+  std::shared_ptr<PinnedPool> pool_ = PinnedPool::get();
 
-  bool open() {
-    if (buf_) return true;
-    if (failed_) return false;
-    bool ok = true;
-    for (auto& e : ev_) ok = ok && (e || hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess);
-    void* p = nullptr;
-    ok = ok && hipHostMalloc(&p, SLOTS * CHUNK, hipHostMallocPortable) == hipSuccess;
-    if (!ok) {
-      (void)hipGetLastError();
-      failed_ = true;
-      return false;
+  // a Pinned of the pool for one copy (where wanted and to be had); every copy
+  // through it has ended when it goes back
+  struct Lease {
+    Lease(HostCopy& h, bool want) : pool(*h.pool_), p(want ? pool.take(h.device) : nullptr) {}
+    ~Lease() {
+      if (p) pool.give(std::move(p));
     }
-    buf_ = static_cast<char*>(p);
-    return true;
-  }
+    explicit operator bool() const { return p != nullptr; }
+    Pinned* operator->() const { return p.get(); }
+    PinnedPool& pool;
+    std::unique_ptr<Pinned> p;
+  };
 };
 
 }  // namespace nflow

@@ -186,6 +186,7 @@ int Batch::open() {
   int dev = 0;
   NFLOW_HIP(hipGetDevice(&dev));
   device = dev;
+  host.device = dev;
   NFLOW_HIP(hipDeviceGetAttribute(&cu_count, hipDeviceAttributeMultiprocessorCount, dev));
   NFLOW_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
   NFLOW_HIP(hipEventCreate(&ev0));
