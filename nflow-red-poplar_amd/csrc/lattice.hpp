@@ -55,6 +55,10 @@ inline FastDiv make_fastdiv(uint32_t d) {
   return r;
 }
 
+// Bits of a solid-mask byte: the node is solid; it is not, but some node one of
+// its links pulls from is.
+enum : int { MASK_SOLID = 1, MASK_BESIDE = 2 };
+
 // One lattice as the kernels see it.  Populations of node n = x + nx*(z + nz*y)
 // live in buf[i] at the element pidx(q, n) of kernels.hip (256-byte runs of
 // consecutive nodes per population); the two buffers and the two side-record
@@ -62,7 +66,7 @@ inline FastDiv make_fastdiv(uint32_t d) {
 struct alignas(16) LatticeDev {
   void* buf[2];
   float* side[2];
-  const uint8_t* mask;  // solid nodes (non-zero), or null
+  const uint8_t* mask;  // solid nodes (MASK_SOLID, MASK_BESIDE), or null
   // Collision counter of the stochastic rounding (CTR_COUNT): a step launch
   // rounds with it plus its own `count` argument; k_init writes the first
   // value, k_advance moves it on.  And the divergence flag (CTR_DIVERGED).
@@ -129,6 +133,10 @@ hipError_t launch_probe(int storage, hipStream_t st, const LatticeDev* d_lats, c
                         int parity);
 // out[i] = divergence flag of lattice i (i < nlat)
 hipError_t launch_flags(hipStream_t st, const LatticeDev* d_lats, int nlat, uint32_t* out);
+// mask as given (non-zero = solid) to the kernels' bits, in place
+hipError_t launch_mask(hipStream_t st, const LatticeDev& L, uint8_t* mask);
+// mask bytes of every row from those of its (y, z), plane[ny][nz]
+hipError_t launch_mask_rows(hipStream_t st, const LatticeDev& L, const uint8_t* plane, uint8_t* mask);
 hipError_t launch_node_type(hipStream_t st, const LatticeDev& L, int* type, int* dirstate);
 hipError_t launch_copy_streams(hipStream_t st, const float* src, float* dst, size_t per_stream, int streams);
 // nblk blocks of 19 runs of 64 floats (the FP32 population layout)

@@ -144,18 +144,24 @@ int lattice_upload_inlet(HostLattice& h, hipStream_t st) {
       const double xi = 2.0 * ((double)(splitmix64(key) >> 11) * (1.0 / 9007199254740992.0)) - 1.0;
       u = (float)(in.inlet_peak * 16.0 * eta * (1.0 - eta) * zeta * (1.0 - zeta) * (1.0 + in.perturb * xi));
     }
-  NFLOW_HIP(hipMemcpyAsync(h.dev.side[0], rec.data(), rec.size() * sizeof(float), hipMemcpyHostToDevice, st));
-  NFLOW_HIP(hipMemcpyAsync(h.dev.side[1], h.dev.side[0], rec.size() * sizeof(float), hipMemcpyDeviceToDevice, st));
   std::vector<uint8_t> m;
   if (in.casetype == NFLOW_PIPE) {  // keSetNodeType, kernel.cu:1078-1094
-    m.resize((size_t)h.dev.n);
+    // the pipe is the same along x: its (y, z) plane goes up, by way of the
+    // side records that are filled next, and is spread over the rows there
+    auto solid = [&](int y, int z) { return y >= 0 && y < in.ny && z >= 0 && z < in.nz && pipe_solid(in, y, z); };
+    m.resize((size_t)in.ny * in.nz);
     for (int y = 0; y < in.ny; ++y)
       for (int z = 0; z < in.nz; ++z) {
-        const uint8_t s = pipe_solid(in, y, z) ? 1 : 0;
-        std::memset(&m[(size_t)in.nx * ((size_t)z + (size_t)in.nz * y)], s, (size_t)in.nx);
+        bool beside = false;
+        for (int k = 0; k < 9; ++k) beside = beside || solid(y + k / 3 - 1, z + k % 3 - 1);
+        m[(size_t)y * in.nz + z] = solid(y, z) ? MASK_SOLID : beside ? MASK_BESIDE : 0;
       }
-    NFLOW_HIP(hipMemcpyAsync(const_cast<uint8_t*>(h.dev.mask), m.data(), m.size(), hipMemcpyHostToDevice, st));
+    uint8_t* plane = reinterpret_cast<uint8_t*>(h.dev.side[0]);
+    NFLOW_HIP(hipMemcpyAsync(plane, m.data(), m.size(), hipMemcpyHostToDevice, st));
+    NFLOW_HIP(launch_mask_rows(st, h.dev, plane, const_cast<uint8_t*>(h.dev.mask)));
   }
+  NFLOW_HIP(hipMemcpyAsync(h.dev.side[0], rec.data(), rec.size() * sizeof(float), hipMemcpyHostToDevice, st));
+  NFLOW_HIP(hipMemcpyAsync(h.dev.side[1], h.dev.side[0], rec.size() * sizeof(float), hipMemcpyDeviceToDevice, st));
   NFLOW_HIP(hipStreamSynchronize(st));
   return 0;
 }
@@ -1065,6 +1071,7 @@ extern "C" int nflow_set_solid_mask(nflow_solver* s, const unsigned char* mask) 
     h.dev.mask = static_cast<const uint8_t*>(h.mask_mem);
   }
   NFLOW_HIP(hipMemcpy(const_cast<uint8_t*>(h.dev.mask), mask, (size_t)h.dev.n, hipMemcpyHostToDevice));
+  NFLOW_HIP(launch_mask(b.stream, h.dev, const_cast<uint8_t*>(h.dev.mask)));
   return 0;
 }
 
