@@ -66,6 +66,8 @@ class Batch {
   size_t d_sweep_cap = 0;
   int nsweep = 0;
   bool sweep_channel = false, sweep_runs = false;
+  // nodes of the largest lattice where all fit k_small (and it is chosen), else 0
+  uint32_t small = 0;
   bool tables_dirty = true;
   bool masked = false;  // some lattice has solid nodes: step with the masked kernel
   bool sr_any = false;  // some lattice rounds its 16-bit stores stochastically

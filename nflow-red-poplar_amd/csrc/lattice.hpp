@@ -101,7 +101,19 @@ struct alignas(16) SweepItem {
   int lat, x0, z0, ya, tx, tz, h, pad;
 };
 
+// k_small: whole lattices of up to SMALL_NODES nodes in a workgroup's LDS.  One
+// compute unit's work per step meets the launch it saves near 2,000 nodes: us
+// per step of one step per launch / k_small, MRT, 512 nodes 3.8 / 1.2, 1000 4.0
+// / 1.75, 1100 4.0 / 2.3, 1728 4.1 / 3.1, 2028 4.1 / 3.8, 2048 in a row 3.65 /
+// 3.8.
+enum : int { SMALL_NT = 1024, SMALL_NODES = 1920 };
+
 // Kernel launchers (kernels.hip).
+// `steps` steps in one launch (k_small) of nlat FP32 cavities without solid
+// nodes, of at most `most` <= SMALL_NODES nodes each: reads buf[parity ^
+// parity0]; the newest state goes to the buffer that as many single steps
+// would leave it in, the one before it to the other.
+hipError_t launch_small(hipStream_t st, const LatticeDev* d_lats, int nlat, uint32_t most, int parity, int steps);
 // masked: use the instantiation that honours LatticeDev::mask (any lattice of
 // the launch has solid nodes); sr: the one that can round stochastically (any
 // lattice of the launch has LatticeDev::sr set), with collision count ctr[0] +

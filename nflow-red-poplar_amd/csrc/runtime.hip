@@ -346,6 +346,16 @@ int Batch::upload_tables() {
     NFLOW_HIP(hipMemcpy(d_lats, devs.data(), devs.size() * sizeof(LatticeDev), hipMemcpyHostToDevice));
   if (!items.empty())
     NFLOW_HIP(hipMemcpy(d_items, items.data(), items.size() * sizeof(WorkItem), hipMemcpyHostToDevice));
+  // whole lattices in LDS, many steps per launch: where every lattice fits
+  small = 0;
+  if (tuning.temporal < 0 && storage == NFLOW_STORAGE_F32)
+    for (const auto& h : lats) {
+      small = h.in.casetype == NFLOW_CAVITY && !h.dev.mask ? std::max(small, h.dev.n) : SMALL_NODES + 1;
+      if (small > SMALL_NODES) {
+        small = 0;
+        break;
+      }
+    }
   const std::vector<SweepItem> sw = sweep_items(tuning);
   nsweep = 0;
   sweep_channel = false;
@@ -428,6 +438,13 @@ int Batch::launch_steps(int nsteps) {
   const bool end_single = read_back;
   read_back = false;
   bool pair_last = false;
+  while (small > 0 && left > 0) {
+    const int k = std::min(left, 4096);  // a launch of some ms at most
+    NFLOW_HIP(launch_small(stream, d_lats, (int)lats.size(), small, gparity, k));
+    gparity ^= k & 1;
+    left -= k;
+    ++launches;
+  }
   if (nsweep > 0 && left >= 2) {
     const int pairs = (left % 2 || end_single) ? (left - 1) / 2 : left / 2;
     for (int k = 0; k < pairs; ++k) {
