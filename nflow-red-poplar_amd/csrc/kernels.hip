@@ -771,9 +771,12 @@ __global__ void __launch_bounds__(256) k_advance(const LatticeDev* __restrict__ 
 // idle.  Measured (us per step, one step per launch / the two-node sweep /
 // this one): 256^3 432 / 254 / 229, 4.5 TB/s x 2; 128^3 55 / 55 / 33.8; 96^3
 // 25.6 / 25.6 / 16.6; 101 x 67 x 83 19.1 / 19.1 / 13.6; 512^3 3701 / 2067 /
-// 1816; channels 512 x 128 x 128 215 / 153 / 132 and 676 x 128 x 128 298 /
+// 1816; channels 512 x 128 x 128 215 / 153 / 125 and 676 x 128 x 128 298 /
 // 268 / 232.  At 256^3 a plane takes 6.9 us, against 6.3 us for its bytes at
-// the layout's copy rate.  16-bit storage does not gain: there the collision,
+// the layout's copy rate; DRAM traffic is 2.7% above one read and one write.
+// (The halo's loads issued along with the own nodes', a plane ahead, run 7%
+// slower, 18% at 192^3: they then miss the lines that the neighbouring tile is
+// about to bring into L2.)  16-bit storage does not gain: there the collision,
 // the conversions and the halo's share of them bind (256^3 FP16 with
 // stochastic rounding 244 us against 216 for one step per launch).
 // ---------------------------------------------------------------------------
@@ -833,30 +836,32 @@ __global__ void __launch_bounds__(SWEEP_NT) k_sweep(const LatticeDev* __restrict
   const uint32_t bn = ((uint32_t)max(ya - 2, 0) * (uint32_t)L.nxz) & ~(B - 1);
   const GPops<T, false> in{static_cast<T*>(L.buf[p]) + window<T>(bn)};
   const GPops<T> out{static_cast<T*>(L.buf[p ^ 1]) + window<T>(bn)};
-  const int t = threadIdx.x;
-  // own node: (x0 + lx, z0 + lz)
-  const int lz = t / txn, lx = t - lz * txn;
+  // What a thread keeps of its place over the sweep: its own node (x0 + lx,
+  // z0 + lz) and its number t.  The loop makes them opaque, so that the
+  // coordinates, addresses and wall tests that follow from them are formed
+  // where they are used: hoisted out of the loop they spilled (76 bytes of
+  // scratch and 795 v_readlane), and a reload waits for every load in flight.
+  int t = threadIdx.x, lz = t / txn, lx = t - lz * txn;
   const bool own_in = lz < tzn;
-  int ox = x0 + lx, oz = z0 + lz;
-  // this thread's halo node: row z0 - 1, row z0 + tzn (x from xa to xb),
-  // column x0 - 1, column x0 + txn, each where inside the box
+  // halo nodes: row z0 - 1, row z0 + tzn (x from xa to xb), column x0 - 1,
+  // column x0 + txn, each where inside the box, one per thread
   const int xa = max(x0 - 1, 0), xb = min(x0 + txn, L.nx - 1), rowlen = xb - xa + 1;
   const int nlo = z0 > 0 ? rowlen : 0, nhi = z0 + tzn < L.nz ? rowlen : 0;
   const int nxl = x0 > 0 ? tzn : 0, nxr = x0 + txn < L.nx ? tzn : 0;
   const bool halo_in = t < nlo + nhi + nxl + nxr;
-  int hx, hz, kind;  // kind 0: row z0 - 1, 1: row z0 + tzn, 2: column x0 - 1, 3: column x0 + txn
-  if (t < nlo) { hx = xa + t; hz = z0 - 1; kind = 0; }
-  else if (t < nlo + nhi) { hx = xa + (t - nlo); hz = z0 + tzn; kind = 1; }
-  else if (t < nlo + nhi + nxl) { hx = x0 - 1; hz = z0 + (t - nlo - nhi); kind = 2; }
-  else { hx = x0 + txn; hz = z0 + (t - nlo - nhi - nxl); kind = 3; }
+  struct Halo {
+    int x, z, kind;  // kind 0: row z0 - 1, 1: row z0 + tzn, 2: column x0 - 1, 3: column x0 + txn
+  };
+  auto halo = [&]() -> Halo {
+    if (t < nlo) return {xa + t, z0 - 1, 0};
+    if (t < nlo + nhi) return {xa + (t - nlo), z0 + tzn, 1};
+    if (t < nlo + nhi + nxl) return {x0 - 1, z0 + (t - nlo - nhi), 2};
+    return {x0 + txn, z0 + (t - nlo - nhi - nxl), 3};
+  };
   // index of node (x, y, z) in the window
   auto node = [&](int x, int y, int z) {
     return (uint32_t)x + (uint32_t)L.nx * ((uint32_t)z + (uint32_t)L.nz * (uint32_t)y) - bn;
   };
-  const int o0 = own_in ? lz * WX + lx : 0;  // own element of a slot, less one
-  // the halo node's element of its slots (rows: e_z = +1 resp. -1 slots;
-  // columns: e_z <= 0 slots, one row further on for e_z = +1)
-  const int h0 = (kind == 0 ? 0 : (kind == 1 ? tzn : hz - z0) * WX) + hx - x0 + 1;
   T raw[Q];
   auto issue = [&](int x, int y, int z, T r[Q]) {
     const uint32_t n = node(x, y, z);
@@ -896,6 +901,7 @@ __global__ void __launch_bounds__(SWEEP_NT) k_sweep(const LatticeDev* __restrict
   };
   // does the link of q at the own node on plane y leave the box?
   auto gone = [&](int q, int y) {
+    const int ox = x0 + lx, oz = z0 + lz;
     return (EX[q] > 0 && ox == 0) || (EX[q] < 0 && ox == L.nx - 1) || (EY[q] > 0 && y == 0) ||
            (EY[q] < 0 && y == L.ny - 1) || (EZ[q] > 0 && oz == 0) || (EZ[q] < 0 && oz == L.nz - 1);
   };
@@ -906,31 +912,35 @@ __global__ void __launch_bounds__(SWEEP_NT) k_sweep(const LatticeDev* __restrict
 #pragma unroll
   for (int q = 0; q < Q; ++q) fp[q] = fc[q] = fn[q] = (T)0.0f;
   // side records: thread t holds float t mod 8 of row z0 - 1 + t / 8
-  const int sz = z0 - 1 + (t >> 3);
-  const bool side_in = CH && L.casetype != CASE_CAVITY && t < (tzn + 2) * 8 && sz >= 0 && sz < L.nz;
+  auto side_in = [&] {
+    const int sz = z0 - 1 + (t >> 3);
+    return L.casetype != CASE_CAVITY && t < (tzn + 2) * 8 && sz >= 0 && sz < L.nz;
+  };
   auto side_load = [&](int y) {
-    const int k = t & 7;
+    const int k = t & 7, sz = z0 - 1 + (t >> 3);
     const int at = k < 2 ? SIDE_RHO + k : k < 5 ? SIDE_U0 + k - 2 : SIDE_U1 + k - 5;
     return ((gptr<const float>)L.side[p])[(size_t)(y * L.nz + sz) * SIDE_REC + at];
   };
   if constexpr (CH) {
-    if (side_in) sidepre[max(ya - 1, 0) & 1][t >> 3][t & 7] = side_load(max(ya - 1, 0));
+    if (side_in()) sidepre[max(ya - 1, 0) & 1][t >> 3][t & 7] = side_load(max(ya - 1, 0));
     __syncthreads();
   }
-  if (own_in) issue(ox, max(ya - 1, 0), oz, raw);
+  if (own_in) issue(x0 + lx, max(ya - 1, 0), z0 + lz, raw);
   for (int yi = ya - 1; yi <= yb; ++yi) {
     const bool plane = yi >= 0 && yi < L.ny;
-    // element of the own node in this plane's half of the exchange, less one;
-    // opaque, so that the addresses and wall tests derived from it and from
-    // the coordinates are formed in the loop and not kept across it
-    int c0 = (yi & 1) * LN + o0, ch = (yi & 1) * LN + h0;
-    asm volatile("" : "+v"(c0), "+v"(ch), "+v"(ox), "+v"(oz));
+    asm volatile("" : "+v"(t), "+v"(lx), "+v"(lz));
+    const int ox = x0 + lx, oz = z0 + lz;
+    // element of the own node in this plane's half of the exchange, less one
+    const int c0 = (yi & 1) * LN + lz * WX + lx;
     if (plane) {
       T rh[Q];
       float sv = 0.0f;
       if constexpr (CH)
-        if (side_in && yi + 1 < L.ny) sv = side_load(yi + 1);
-      if (halo_in) issue(hx, yi, hz, rh);
+        if (side_in() && yi + 1 < L.ny) sv = side_load(yi + 1);
+      if (halo_in) {
+        const Halo h = halo();
+        issue(h.x, yi, h.z, rh);
+      }
       if (own_in) {
         T e[Q];
         step1(raw, ox, yi, oz, e);
@@ -945,17 +955,22 @@ __global__ void __launch_bounds__(SWEEP_NT) k_sweep(const LatticeDev* __restrict
       }
       asm volatile("" ::: "memory");  // the halo node's arithmetic after the own node's: registers
       if (halo_in) {
+        asm volatile("" : "+v"(t));
+        const Halo h = halo();
         T e[Q];
-        step1(rh, hx, yi, hz, e);
-        if (kind == 0) {
+        step1(rh, h.x, yi, h.z, e);
+        // its element of its slots (rows: e_z = +1 resp. -1 slots; columns:
+        // e_z <= 0 slots, one row further on for e_z = +1)
+        const int ch = (yi & 1) * LN + (h.kind == 0 ? 0 : (h.kind == 1 ? tzn : h.z - z0) * WX) + h.x - x0 + 1;
+        if (h.kind == 0) {
 #pragma unroll
           for (int q = 0; q < Q; ++q)
             if (EZ[q] > 0) cross[ch + base_of(slot_of(q))] = e[q];
-        } else if (kind == 1) {
+        } else if (h.kind == 1) {
 #pragma unroll
           for (int q = 0; q < Q; ++q)
             if (EZ[q] < 0) cross[ch + base_of(slot_of(q))] = e[q];
-        } else if (kind == 2) {
+        } else if (h.kind == 2) {
 #pragma unroll
           for (int q = 0; q < Q; ++q)
             if (EX[q] > 0) cross[(EZ[q] > 0 ? ch + WX : ch) + base_of(slot_of(q))] = e[q];
@@ -967,7 +982,7 @@ __global__ void __launch_bounds__(SWEEP_NT) k_sweep(const LatticeDev* __restrict
       }
       asm volatile("" ::: "memory");  // and the next plane's loads after both
       if constexpr (CH)
-        if (side_in) sidepre[(yi + 1) & 1][t >> 3][t & 7] = sv;
+        if (side_in()) sidepre[(yi + 1) & 1][t >> 3][t & 7] = sv;
       if (own_in && yi < yb && yi + 1 < L.ny) issue(ox, yi + 1, oz, raw);
     }
     __syncthreads();

@@ -731,7 +731,7 @@ struct SweepShape {
 // One workgroup fills a CU (its LDS).  It sweeps its h planes, plus 0.28 for
 // the planes around the chunk that it only takes the first step on, at
 //   3.58 + 0.22 halo + w (3.06 fill m + x) us a plane
-// (x 1.14 for channels), halo and fill the halo and own nodes per thread, m =
+// (x 1.05 for channels), halo and fill the halo and own nodes per thread, m =
 // 1.32 where rows do not start on 128-byte lines, x = 0.97 for tiles split in
 // x, 2.04 where the splits are off 64-byte boundaries, and 3.1 us for its
 // start.  Fitted, with 4 us a launch and 6% for more than one round of
@@ -747,7 +747,7 @@ static SweepShape sweep_shape(const nflow_input& in, int tx, int tz, int h) {
   s.wgs = (long)ntx * ntz * nch;
   const double halo = ((ntz > 1 ? 2.0 * (tx + 2) : 0.0) + (ntx > 1 ? 2.0 * tz : 0.0)) / SWEEP_NT;
   const double fill = (double)tx * tz / SWEEP_NT, split = ntx == 1 ? 0.0 : tx % 16 ? 2.04 : 0.97;
-  const double planes = ((double)in.ny / nch + 0.28) * (in.casetype == NFLOW_CHANNEL ? 1.14 : 1.0);
+  const double planes = ((double)in.ny / nch + 0.28) * (in.casetype == NFLOW_CHANNEL ? 1.05 : 1.0);
   s.us0 = 3.1 + planes * (3.58 + 0.22 * halo);
   s.us1 = planes * (3.06 * fill * (in.nx % 32 ? 1.32 : 1.0) + split);
   return s;
