@@ -76,8 +76,13 @@ class Batch {
   // step launches since the lattices' collision counters were last moved on:
   // the count argument of the next one
   uint32_t count = 0;
-  hipGraphExec_t graph[2] = {nullptr, nullptr};
+  // captured steps by starting parity: tuning.graph_steps of them, and
+  // LONG_GRAPH times as many once the short graphs have been replayed
+  // LONG_AFTER times
+  static constexpr int LONG_GRAPH = 10, LONG_AFTER = 30;
+  hipGraphExec_t graph[2] = {nullptr, nullptr}, long_graph[2] = {nullptr, nullptr};
   int graph_steps_built = 0;
+  int replays = 0;  // of the short graphs
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   int last_steps = 0;
   long long launches = 0;
@@ -144,7 +149,7 @@ class Batch {
 
  private:
   int ensure_scratch(size_t aos, size_t macro, size_t partials, size_t types);
-  int build_graph(int parity);
+  int build_graph(hipGraphExec_t* out, int parity, int steps);
 };
 
 }  // namespace nflow

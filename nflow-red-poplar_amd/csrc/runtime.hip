@@ -239,15 +239,17 @@ void Batch::remove_lattice(int idx) {
 // An executable graph may still be running on the stream (its replays are
 // only enqueued), so the stream drains before the graphs are destroyed.
 void Batch::destroy_graphs() {
+  hipGraphExec_t* const all[] = {&graph[0], &graph[1], &long_graph[0], &long_graph[1]};
   bool any = false;
-  for (auto& g : graph) any = any || g != nullptr;
+  for (auto* g : all) any = any || *g != nullptr;
   if (any && stream) (void)hipStreamSynchronize(stream);
-  for (auto& g : graph)
-    if (g) {
-      (void)hipGraphExecDestroy(g);
-      g = nullptr;
+  for (auto* g : all)
+    if (*g) {
+      (void)hipGraphExecDestroy(*g);
+      *g = nullptr;
     }
   graph_steps_built = 0;
+  replays = 0;
 }
 
 long long Batch::total_nodes() const {
@@ -399,26 +401,24 @@ int Batch::init_all() {
   return 0;
 }
 
-int Batch::build_graph(int parity) {
+int Batch::build_graph(hipGraphExec_t* out, int parity, int steps) {
   hipGraph_t g = nullptr;
   NFLOW_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
   int p = parity;
   hipError_t err = hipSuccess;
-  for (int s = 0; s < tuning.graph_steps && err == hipSuccess; ++s) {
+  for (int s = 0; s < steps && err == hipSuccess; ++s) {
     err = launch_step(storage, masked, sr_any, tuning.block, grid, stream, d_lats, d_items, nitems, p, (uint32_t)s);
     p ^= 1;
   }
-  if (sr_any && err == hipSuccess)
-    err = launch_advance(stream, d_lats, (int)lats.size(), (uint32_t)tuning.graph_steps);
+  if (sr_any && err == hipSuccess) err = launch_advance(stream, d_lats, (int)lats.size(), (uint32_t)steps);
   hipError_t e2 = hipStreamEndCapture(stream, &g);
   if (err != hipSuccess || e2 != hipSuccess) {
     if (g) (void)hipGraphDestroy(g);
     return fail(NFLOW_EDEVICE, "graph capture failed: %s", hipGetErrorString(err != hipSuccess ? err : e2));
   }
-  hipError_t e3 = hipGraphInstantiate(&graph[parity], g, nullptr, nullptr, 0);
+  hipError_t e3 = hipGraphInstantiate(out, g, nullptr, nullptr, 0);
   (void)hipGraphDestroy(g);
   if (e3 != hipSuccess) return fail(NFLOW_EDEVICE, "hipGraphInstantiate: %s", hipGetErrorString(e3));
-  graph_steps_built = tuning.graph_steps;
   return 0;
 }
 
@@ -459,16 +459,28 @@ int Batch::launch_steps(int nsteps) {
   if (gs > 0 && left >= gs && nitems > 0) {
     if (graph_steps_built != gs) destroy_graphs();
     if (!graph[gparity]) {
-      rc = build_graph(gparity);
+      rc = build_graph(&graph[gparity], gparity, gs);
       if (rc) return rc;
+      graph_steps_built = gs;
     }
-    const int reps = left / gs;
     // a replay's launches count from 0
     if (sr_any && count) NFLOW_HIP(launch_advance(stream, d_lats, (int)lats.size(), count));
     count = 0;
-    for (int r = 0; r < reps; ++r) NFLOW_HIP(hipGraphLaunch(graph[gparity], stream));
-    left -= reps * gs;
-    launches += (long long)reps * gs;
+    // the GPU idles for some 7 us between replays: 48^3 FP16 runs at 5.7 us
+    // per step in graphs of 10 steps and 5.0 in graphs of 100, which take ten
+    // times as long to build, so they come once the short ones have been used
+    const int ls = LONG_GRAPH * gs;
+    if (replays >= LONG_AFTER && left >= ls && gs <= 100) {
+      if (!long_graph[gparity]) {
+        rc = build_graph(&long_graph[gparity], gparity, ls);
+        if (rc) return rc;
+      }
+      launches += left / ls * ls;
+      for (; left >= ls; left -= ls) NFLOW_HIP(hipGraphLaunch(long_graph[gparity], stream));
+    }
+    launches += left / gs * gs;
+    replays = std::min(replays + left / gs, LONG_AFTER);
+    for (; left >= gs; left -= gs) NFLOW_HIP(hipGraphLaunch(graph[gparity], stream));
   }
   for (int s = 0; s < left; ++s) {
     NFLOW_HIP(launch_step(storage, masked, sr_any, tuning.block, grid, stream, d_lats, d_items, nitems, gparity, count));
