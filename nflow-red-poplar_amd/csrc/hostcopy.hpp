@@ -4,10 +4,11 @@
 // The caller's arrays are pageable and often fresh, so a plain copy is bound
 // by one thread taking their page faults: 256 MiB into a new array took 27 ms
 // (10 GB/s) with a 57 GB/s link, 1 MiB 0.63 ms.  Here the link fills pinned
-// chunks and up to eight threads move them on, so that the faults and the
+// chunks and four threads move them on, so that the faults and the
 // copies overlap with the link: 6.3-6.9 ms (39-42 GB/s), 64 MiB 7.4 -> 1.95
 // ms, 9 MiB 0.89 -> 0.40 ms.  Chunks of 1 MiB reached 31 GB/s, of 2 and 4 MiB
-// 39-42; four threads are as good as twelve for 256 MiB, eight best at 9 MiB.
+// 39-42.  More than four threads gain 0 to 6%, and after eight the next
+// solver's creation took 110 or, one time in three, 400 to 900 us.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -42,13 +43,21 @@ void run_threads(int extra, F f, Main mine) {
   for (int i = 0; i < n; ++i) t[i].join();
 }
 
-// Helpers for a copy; 0: too small for threads.  From 3 MiB eight of them
-// halve the time into fresh pages (8 MiB 1.9 -> 0.9 ms), and lose little where
-// malloc hands the same pages out again (0.5 -> 0.7 ms).  1.7 MiB is 130 us as
-// the runtime's own pageable copies, 310 us through the chunks.
-inline int copy_threads(size_t bytes) {
+// Helpers for a copy into the caller's pages; 0: too small for threads.  From
+// 3 MiB they halve the time into fresh pages (8 MiB 1.9 -> 0.9 ms), and lose
+// little where malloc hands the same pages out again (0.5 -> 0.7 ms).  1.7 MiB
+// is 130 us as the runtime's own pageable copies, 310 us through the chunks.
+inline int helpers_out(size_t bytes) {
   const unsigned hw = std::thread::hardware_concurrency();
-  return bytes < (3u << 20) ? 0 : (int)std::min<size_t>({bytes >> 19, 8, hw ? hw : 1});
+  return bytes < (3u << 20) ? 0 : (int)std::min<size_t>(3, hw ? hw : 1);
+}
+
+// Helpers for a copy out of the caller's pages, which mostly are there: 67 MB
+// 2.6 -> 2.0 ms, but 9.5 MB 300 us as the runtime's own copy and 370 to 750
+// through the chunks.
+inline int helpers_in(size_t bytes) {
+  const unsigned hw = std::thread::hardware_concurrency();
+  return bytes < (32u << 20) ? 0 : (int)std::min<size_t>(8, hw ? hw : 1);
 }
 
 // memcpy by several threads (fresh destination pages are faulted in by all)
@@ -59,7 +68,7 @@ inline void parallel_memcpy(void* dst, const void* src, size_t n) {
     for (size_t o; (o = next.fetch_add(PIECE)) < n;)
       std::memcpy(static_cast<char*>(dst) + o, static_cast<const char*>(src) + o, std::min(PIECE, n - o));
   };
-  run_threads(copy_threads(n), work, [&](int) { work(); });
+  run_threads(helpers_out(n), work, [&](int) { work(); });
 }
 
 // Pinned chunks and the events of the copies through them.
@@ -136,7 +145,7 @@ class HostCopy {
   // dst[1], ...; complete on return, and so is all earlier work of the stream.
   int to_host(hipStream_t st, const void* src, size_t n, void* const* dst, int parts) {
     const size_t total = n * parts;
-    const int helpers = copy_threads(total);
+    const int helpers = helpers_out(total);
     const Lease lease(*this, helpers > 0 || total <= SMALL);
     if (!lease) {  // plain copies
       for (int i = 0; i < parts; ++i)
@@ -226,7 +235,8 @@ class HostCopy {
   // n bytes from the host to dst on the device, in stream order; src may be
   // reused on return (the last chunks may still be on their way).
   int to_device(hipStream_t st, void* dst, const void* src, size_t n) {
-    const Lease lease(*this, copy_threads(n) > 0);
+    const int most = helpers_in(n);
+    const Lease lease(*this, most > 0);
     if (!lease) {
       NFLOW_HIP(hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, st));
       NFLOW_HIP(hipStreamSynchronize(st));
@@ -255,7 +265,7 @@ class HostCopy {
       }
     };
     hipError_t err = hipSuccess;
-    run_threads(copy_threads(n), work, [&](int helpers) {
+    run_threads(most, work, [&](int helpers) {
       for (size_t c = 0; c < chunks && err == hipSuccess; ++c) {
         // chunk c - SLOTS / 2 has left: its slot may be filled again
         if (c >= SLOTS / 2) {

@@ -1099,8 +1099,9 @@ extern "C" int nflow_set_solid_mask(nflow_solver* s, const unsigned char* mask) 
     }
     h.dev.mask = static_cast<const uint8_t*>(h.mask_mem);
   }
-  NFLOW_HIP(hipMemcpy(const_cast<uint8_t*>(h.dev.mask), mask, (size_t)h.dev.n, hipMemcpyHostToDevice));
+  NFLOW_HIP(hipMemcpyAsync(const_cast<uint8_t*>(h.dev.mask), mask, (size_t)h.dev.n, hipMemcpyHostToDevice, b.stream));
   NFLOW_HIP(launch_mask(b.stream, h.dev, const_cast<uint8_t*>(h.dev.mask)));
+  NFLOW_HIP(hipStreamSynchronize(b.stream));  // the caller's array may go
   return 0;
 }
 

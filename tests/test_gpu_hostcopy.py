@@ -1,7 +1,7 @@
 """Copies between device memory and the caller's arrays (csrc/hostcopy.hpp):
 populations written and read back unchanged at sizes on either side of the
-plain, single and chunked paths (1 MiB, 3 MiB), of one chunk (2 MiB) and of
-all eight (16 MiB, where chunks are used again), into views that start off any
+plain, single and chunked paths (1 and 3 MiB out, 32 MiB in), of one chunk (2
+MiB) and of all eight (16 MiB, where chunks are used again), into views that start off any
 boundary; and from two host threads at once."""
 import threading
 
