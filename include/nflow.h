@@ -203,7 +203,7 @@ typedef struct nflow_tuning {
   int block;       /* threads per workgroup: 64, 128, 256 or 512 */
   int xcd_order;   /* 1: each XCD receives a contiguous range of work items */
   int persistent;  /* 0: one workgroup per work item; k > 0: k workgroups per CU, grid-stride */
-  int graph_steps; /* steps per captured graph (even), 0 = no graph */
+  int graph_steps; /* steps per captured graph (even), 0 = no graph; batches in longer use replay ten times as many */
   /* Two steps per launch for FP32 cavities and channels without solid nodes
    * (other batches ignore this), in x-z tiles swept along y in chunks of H
    * planes, with results bit for bit those of one step per launch.  A run of
