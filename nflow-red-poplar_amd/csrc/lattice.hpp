@@ -4,6 +4,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "sweep_plan.hpp"
+
 namespace nflow {
 
 enum : int { CASE_PIPE = 0, CASE_CAVITY = 1, CASE_CHANNEL = 2 };  // NFLOW_PIPE/CAVITY/CHANNEL
@@ -88,17 +90,6 @@ struct alignas(16) WorkItem {
   uint32_t start;
   uint32_t count;
   uint32_t pad;
-};
-
-// Work of one workgroup of k_sweep (two steps per launch): a tile of tx x tz
-// nodes of the x-z plane from (x0, z0), one per thread (tx tz <= SWEEP_NT, tz
-// <= SWEEP_ROWS), swept over the y planes [ya, ya + h); h = 0: no work.  The
-// exchange between the columns holds, per crossing population, SWEEP_SLOT0
-// elements where e_z = 0, at least tz (tx + 2), and SWEEP_SLOT1 where it is
-// not, at least (tz + 1) (tx + 2); two planes of it fill the LDS.
-enum : int { SWEEP_NT = 1024, SWEEP_ROWS = 32, SWEEP_SLOT0 = 1088, SWEEP_SLOT1 = 1296 };
-struct alignas(16) SweepItem {
-  int lat, x0, z0, ya, tx, tz, h, pad;
 };
 
 // k_small: whole lattices of up to SMALL_NODES nodes in a workgroup's LDS.  One

@@ -1,0 +1,74 @@
+"""The choice of two steps per launch, its tiles and its chunk heights
+(csrc/sweep_plan.cpp), without a GPU: the driver checks every work list against
+the kernel's limits; here, which lattices get one."""
+import os
+import random
+import shutil
+import subprocess
+
+import pytest
+
+import nflow
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CAV, CH = nflow.CAVITY, nflow.CHANNEL
+
+
+@pytest.fixture(scope="module")
+def plan(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("g++ not installed")
+    exe = str(tmp_path_factory.mktemp("plan") / "driver")
+    csrc = os.path.join(ROOT, "nflow-red-poplar_amd", "csrc")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-I", os.path.join(ROOT, "include"), "-I", csrc,
+                    os.path.join(ROOT, "tests", "sweep_plan_driver.cpp"), os.path.join(csrc, "sweep_plan.cpp"),
+                    "-o", exe], check=True)
+
+    def run(lats, temporal=-1, cus=256):
+        r = subprocess.run([exe, str(cus), str(temporal)] + [str(v) for s in lats for v in s], capture_output=True,
+                           text=True, timeout=60)
+        assert r.returncode == 0, (lats, temporal, r.stderr)
+        return None if r.stdout == "none\n" else [tuple(map(int, w.split())) for w in r.stdout.splitlines()]
+
+    return run
+
+
+LARGE = [(576, 576, 576, CAV), (600, 600, 600, CAV), (640, 640, 640, CAV), (768, 768, 768, CAV),
+         (1024, 1024, 1024, CAV), (1200, 1200, 1200, CAV), (512, 1600, 512, CAV), (984, 52, 1039, CAV),
+         (1024, 512, 512, CH), (2048, 256, 256, CH), (2048, 512, 512, CH), (4096, 256, 256, CH), (2000, 20, 2500, CAV)]
+
+
+@pytest.mark.parametrize("shape", LARGE)
+def test_large_planes_take_chunks_that_a_window_holds(plan, shape):
+    """The tiles of one plane are as many as the CUs: chunks for up to five
+    rounds of the CUs are taller than 32-bit offsets reach."""
+    (_, _, h, _), = plan([shape])
+    most = ((2 ** 32 - 1) // 76 - 64) // (shape[0] * shape[2]) - 4
+    assert 1 <= h <= most
+    assert h == shape[1] or h > most // 2
+    # in a batch too, and beside a lattice that fits as it is
+    assert plan([shape, shape]) and plan([(128, 128, 128, CAV), shape])
+    # a height that does not fit stays refused
+    assert plan([shape], temporal=most) and plan([shape], temporal=most + 1) is None
+
+
+def test_any_box_within_the_kernel_limits(plan):
+    rng = random.Random(1)
+    for k in range(150):
+        d = [int(2 ** rng.uniform(0, 10.5)) for _ in range(3)]
+        lat = (*d, CH if rng.random() < 0.5 and d[0] > 2 else CAV)
+        h = int(2 ** rng.uniform(0, 12))
+        if d[0] * d[1] * d[2] < 2e9:
+            plan([lat])
+            plan([lat], temporal=h)
+            plan([lat, (90, 80, 70, CAV)])
+
+
+def test_not_where_it_does_not_apply(plan):
+    big = (256, 256, 256, CAV)
+    assert plan([big]) and plan([big], temporal=24)[0][2] == 24
+    assert plan([big], temporal=0) is None
+    assert plan([(256, 256, 256, nflow.PIPE)]) is None and plan([big, (256, 256, 256, nflow.PIPE)]) is None
+    assert plan([big, big], temporal=16) is None  # a height is a choice for one lattice
+    assert plan([(48, 48, 48, CAV)]) is None
+    assert plan([(3700, 8, 3700, CAV)]) is None  # not a plane fits a window
