@@ -8,10 +8,12 @@
 
 namespace nflow {
 
-// A workgroup of k_sweep reads planes ya - 2 .. ya + h + 1, rounded down to a
-// block of 64 nodes, through a window of 32-bit byte offsets.
+// A workgroup of k_sweep reads planes ya - 2 .. ya + h + 1 through a window of
+// 32-bit byte offsets that starts at the first plane's block of 64 nodes: its
+// farthest element is run 18 of node (h + 4) nxz + 62 of the window, 19 (h + 4)
+// nxz + 19 x 62 + 18 x 64 at most.
 int sweep_max_height(const nflow_input& in) {
-  constexpr long long nodes = ((1ll << 32) - 1) / (19 * 4) - 64;
+  constexpr long long nodes = ((1ll << 30) - 1 - 19 * 62 - 18 * 64) / 19;
   return (int)std::max(0ll, nodes / ((long long)in.nx * in.nz) - 4);
 }
 

@@ -3,6 +3,7 @@
 // nx ny nz casetype per lattice.  Prints "tx tz h workgroups" per lattice (one
 // line "none" without a plan) after checking the work list: tiles within the
 // kernel's limits, each node in exactly one.
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <vector>
@@ -47,8 +48,11 @@ int main(int argc, char** argv) {
       CHECK(w.tx * w.tz <= SWEEP_NT && w.tz <= SWEEP_ROWS);
       CHECK(w.tz * (w.tx + 2) <= SWEEP_SLOT0 && (w.tz + 1) * (w.tx + 2) <= SWEEP_SLOT1);
       CHECK(2 * (w.tx + 2) + 2 * w.tz <= SWEEP_NT);  // one halo node per thread
-      // its farthest byte: planes ya - 2 .. ya + h + 1 from a block of 64 nodes
-      CHECK(((w.h + 4ll) * l.nx * l.nz + 64) * 19 * 4 < 1ll << 32);
+      // its farthest byte: the last node of planes ya - 2 .. ya + h + 1 in blocks
+      // of 19 runs of 64 nodes, from the block that the first one lies in
+      const long long nxz = (long long)l.nx * l.nz, from = std::max(w.ya - 2, 0) * nxz / 64 * 64;
+      const long long n = std::min<long long>(l.ny, (long long)w.ya + w.h + 2) * nxz - 1 - from;
+      CHECK(((n / 64 * 19 + 18) * 64 + n % 64) * 4 + 3 < 1ll << 32);
       CHECK(w.x0 % s.tx == 0 && w.z0 % s.tz == 0 && w.ya % s.h == 0 && w.x0 < l.nx && w.z0 < l.nz && w.ya < l.ny);
       unsigned char& at = seen[(size_t)(w.x0 / s.tx) + (size_t)((l.nx - 1) / s.tx + 1) *
                                    ((size_t)(w.z0 / s.tz) + (size_t)((l.nz - 1) / s.tz + 1) * (w.ya / s.h))];

@@ -43,13 +43,23 @@ def test_large_planes_take_chunks_that_a_window_holds(plan, shape):
     """The tiles of one plane are as many as the CUs: chunks for up to five
     rounds of the CUs are taller than 32-bit offsets reach."""
     (_, _, h, _), = plan([shape])
-    most = ((2 ** 32 - 1) // 76 - 64) // (shape[0] * shape[2]) - 4
+    most = (2 ** 30 - 2331) // 19 // (shape[0] * shape[2]) - 4
     assert 1 <= h <= most
     assert h == shape[1] or h > most // 2
     # in a batch too, and beside a lattice that fits as it is
     assert plan([shape, shape]) and plan([(128, 128, 128, CAV), shape])
     # a height that does not fit stays refused
     assert plan([shape], temporal=most) and plan([shape], temporal=most + 1) is None
+
+
+def test_windows_that_end_at_32_bits(plan):
+    """Heights whose h + 4 planes come within 59 nodes of what 32-bit byte
+    offsets reach: the first plane starts up to 63 nodes into its block, and
+    the last node's run 18 lies up to 1,152 elements on."""
+    for nx, nz, h in ((1429, 557, 67), (557, 1429, 67), (1847, 1457, 17), (1457, 1847, 17), (2718, 2599, 4)):
+        for below in (0, 1):
+            plan([(nx, 5 * h + 3, nz, CAV)], temporal=h - below)
+        plan([(nx, 5 * h + 3, nz, CAV)])
 
 
 def test_any_box_within_the_kernel_limits(plan):
