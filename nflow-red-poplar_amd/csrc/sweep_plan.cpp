@@ -29,8 +29,8 @@ static int even_height(int ny, int h) {
 // (x 1.05 for channels), halo and fill the halo and own nodes per thread, m =
 // 1.32 where rows do not start on 128-byte lines, x = 0.97 for tiles split in
 // x, 2.04 where the splits are off 64-byte boundaries, and 3.1 us for its
-// start.  Fitted, with 4 us a launch and 6% for more than one round of
-// workgroups, to 600 launches of 62 cavities and channels of 40^3 to 512^3
+// start.  Fitted, with 4 us a launch and SWEEP_ROUNDS for more than one round
+// of workgroups, to 600 launches of 62 cavities and channels of 40^3 to 512^3
 // nodes at up to 18 shapes each (9% rms); the shape it picks is within 1.2% of
 // the fastest measured one on average, and within 12%.
 static SweepShape sweep_shape(const nflow_input& in, int tx, int tz, int h) {
@@ -47,14 +47,34 @@ static SweepShape sweep_shape(const nflow_input& in, int tx, int tz, int h) {
   s.us1 = planes * (3.06 * fill * (in.nx % 32 ? 1.32 : 1.0) + split);
   return s;
 }
-static constexpr double SWEEP_LAUNCH_US = 4.0, SWEEP_ROUNDS = 1.06;
+static constexpr double SWEEP_ROUNDS = 1.06;
 
-// us of one step per launch of one lattice, and 3 us a launch: 39 nodes per
-// ns, 12% less where rows do not start on 128-byte lines
-static double one_step_us(const nflow_input& in) {
-  return (double)in.nx * in.ny * in.nz / 39.0e3 * (in.nx % 32 ? 1.12 : 1.0);
+// Whether two steps in one launch beat two launches is a question of small
+// lattices: chunks of few planes and CUs without work, where the estimate above
+// is up to 7 us short for channels.  For that question alone: us of a workgroup
+// of shape s when w of the CUs are busy, and us of two single steps.  Fitted,
+// with 4 us for the launch, to 900 cavities and channels of 30,000 to 2,000,000
+// nodes near the line (1.6 and 1.9 us rms, two single steps 5%).  On 400 others
+// the answer costs 0.6% against the faster of the two and 8 are more than 2%
+// slower; by the estimate above 3.5%, and 87 were slower, by up to 40%, channels
+// of some 100,000 nodes above all (274 x 28 x 24: 11.2 us a step, and 8.1 with
+// one step per launch).
+static double sweep_wg_us(const nflow_input& in, const SweepShape& s, double w) {
+  const bool ch = in.casetype == NFLOW_CHANNEL;
+  const double halo = ((s.tz < in.nz ? 2.0 * (s.tx + 2) : 0.0) + (s.tx < in.nx ? 2.0 * s.tz : 0.0)) / SWEEP_NT;
+  const double fill = (double)s.tx * s.tz / SWEEP_NT * (in.nx % 32 ? 1.32 : 1.0);
+  const double planes = (double)in.ny / ((in.ny - 1) / s.h + 1) + 0.28;
+  const double plane = ch ? 4.84 + 0.39 * halo + 2.93 * w * fill - (s.tx < in.nx ? 0.18 : 0.0)
+                          : 2.81 + 1.29 * halo + 3.16 * w * fill + (s.tx < in.nx ? 0.21 : 0.0);
+  return (ch ? 4.95 + 4.36 * halo : 2.97 + 4.59 * halo) + planes * plane;
 }
-static constexpr double ONE_STEP_LAUNCH_US = 3.0;
+static double two_steps_us(const nflow_input& in) {
+  const bool ch = in.casetype == NFLOW_CHANNEL;
+  return (double)in.nx * in.ny * in.nz / 39.0e3 * ((ch ? 2.05 : 2.0) + (in.nx % 32 ? 0.14 : 0.0));
+}
+static constexpr double SWEEP_LAUNCH_US = 4.0, TWO_LAUNCHES_US = 5.3;
+// two steps per launch where they gain this much by the estimates
+static constexpr double SWEEP_GAIN = 1.02;
 
 // The candidate tile shapes of a lattice: whole x rows where three of them
 // fit the exchange, and widths of 64-byte multiples; as many rows as fit,
@@ -80,7 +100,7 @@ std::vector<SweepShape> sweep_plan(const std::vector<nflow_input>& lats, int cu_
   for (const auto& in : lats)
     if (in.casetype == NFLOW_PIPE || sweep_max_height(in) < std::max(temporal, 1)) return none;
   std::vector<SweepShape> shape(lats.size());
-  double single = 2.0 * ONE_STEP_LAUNCH_US, pair = SWEEP_LAUNCH_US;  // us of two steps, either way
+  double single = TWO_LAUNCHES_US, pair = SWEEP_LAUNCH_US;  // us of two steps, either way
   if (lats.size() == 1) {
     const nflow_input& in = lats[0];
     double best = 1e30;
@@ -105,8 +125,9 @@ std::vector<SweepShape> sweep_plan(const std::vector<nflow_input>& lats, int cu_
         }
       }
     }
-    single += 2.0 * one_step_us(in);
-    pair += best;
+    const long rounds = (shape[0].wgs - 1) / cu_count + 1;
+    single += two_steps_us(in);
+    pair += rounds * sweep_wg_us(in, shape[0], (double)shape[0].wgs / ((double)rounds * cu_count));
   } else {
     // every CU takes workgroups until none are left: the launch lasts as long
     // as their sum spread over the CUs, plus half of the longest at its end
@@ -134,10 +155,17 @@ std::vector<SweepShape> sweep_plan(const std::vector<nflow_input>& lats, int cu_
         shape = c;
       }
     }
-    for (const auto& in : lats) single += 2.0 * one_step_us(in);
-    pair += best;
+    // (35^3 x 57 channels: 105.5 us a step, and 78.6 with one step per launch)
+    double sum = 0.0, longest = 0.0;
+    for (size_t i = 0; i < lats.size(); ++i) {
+      const double us = sweep_wg_us(lats[i], shape[i], 1.0);
+      sum += shape[i].wgs * us;
+      longest = std::max(longest, us);
+      single += two_steps_us(lats[i]);
+    }
+    pair += sum / cu_count + 0.5 * longest;
   }
-  if (temporal < 0 && pair >= single) return none;
+  if (temporal < 0 && pair * SWEEP_GAIN >= single) return none;
   return shape;
 }
 

@@ -82,3 +82,28 @@ def test_not_where_it_does_not_apply(plan):
     assert plan([big, big], temporal=16) is None  # a height is a choice for one lattice
     assert plan([(48, 48, 48, CAV)]) is None
     assert plan([(3700, 8, 3700, CAV)]) is None  # not a plane fits a window
+
+
+# us per step of one and of two steps per launch, measured on 256 CUs with the
+# tiles and heights that the plan picks
+MEASURED = [
+    ((274, 28, 24, CH), 8.1, 11.2), ((322, 47, 19, CH), 10.7, 14.9), ((142, 12, 110, CH), 7.8, 10.6),
+    ((56, 52, 62, CH), 7.7, 9.7), ((30, 36, 245, CH), 11.5, 13.5), ((211, 5, 181, CH), 7.4, 10.4),
+    ((170, 4, 248, CAV), 7.4, 8.6), ((306, 13, 44, CAV), 8.0, 9.6), ((59, 13, 217, CAV), 6.6, 7.9),
+    ((194, 27, 32, CAV), 6.4, 8.3),
+    ((96, 96, 96, CAV), 25.6, 16.6), ((101, 67, 83, CAV), 17.9, 13.6), ((128, 128, 128, CAV), 53.5, 33.8),
+    ((66, 62, 233, CH), 30.1, 22.7), ((44, 98, 246, CH), 34.2, 24.9), ((512, 128, 128, CH), 215.0, 125.4),
+    ((30, 150, 104, CAV), 16.6, 12.4), ((179, 32, 154, CAV), 26.4, 18.1), ((28, 323, 96, CH), 27.8, 17.1),
+]
+
+
+@pytest.mark.parametrize("lat,one,two", MEASURED)
+def test_two_steps_per_launch_only_where_they_are_faster(plan, lat, one, two):
+    assert (plan([lat]) is not None) == (two < one)
+
+
+def test_batches_take_two_steps_only_where_they_are_faster(plan):
+    assert plan([(35, 35, 35, CH)] * 57) is None  # 78.6 us a step, 105.5 in pairs
+    assert plan([(47, 47, 47, CH)] * 26) is None  # 79.8 and 88.8
+    assert plan([(48, 48, 48, CAV)] * 16)  # 51.7 and 39.4
+    assert plan([(77, 77, 77, CH)] * 6)  # 0.82 of one step's time
