@@ -141,6 +141,8 @@ class Batch {
   // 256 x 8 node tiles, resolving temporal = -1 by an estimate for those; 0:
   // none
   int step2_height(const nflow_tuning* t = nullptr) const;
+  // nodes of the largest lattice where all run in k_small under `t`, else 0
+  uint32_t small_nodes(const nflow_tuning& t) const;
   // work list of two-step launches under `t`, empty for one step per launch
   std::vector<SweepItem> sweep_items(const nflow_tuning& t) const;
   void destroy_graphs();

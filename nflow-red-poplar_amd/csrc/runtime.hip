@@ -349,16 +349,7 @@ int Batch::upload_tables() {
     NFLOW_HIP(hipMemcpy(d_lats, devs.data(), devs.size() * sizeof(LatticeDev), hipMemcpyHostToDevice));
   if (!items.empty())
     NFLOW_HIP(hipMemcpy(d_items, items.data(), items.size() * sizeof(WorkItem), hipMemcpyHostToDevice));
-  // whole lattices in LDS, many steps per launch: where every lattice fits
-  small = 0;
-  if (tuning.temporal < 0 && storage == NFLOW_STORAGE_F32)
-    for (const auto& h : lats) {
-      small = h.in.casetype == NFLOW_CAVITY && !h.dev.mask ? std::max(small, h.dev.n) : SMALL_NODES + 1;
-      if (small > SMALL_NODES) {
-        small = 0;
-        break;
-      }
-    }
+  small = small_nodes(tuning);
   const std::vector<SweepItem> sw = sweep_items(tuning);
   nsweep = 0;
   sweep_channel = false;
@@ -722,6 +713,17 @@ int Batch::step2_height(const nflow_tuning* t) const {
   return best;
 }
 
+// Whole lattices in LDS, many steps per launch (k_small): where every lattice fits.
+uint32_t Batch::small_nodes(const nflow_tuning& t) const {
+  if (t.temporal >= 0 || storage != NFLOW_STORAGE_F32) return 0;
+  uint32_t most = 0;
+  for (const auto& h : lats) {
+    if (h.in.casetype != NFLOW_CAVITY || h.dev.mask || h.dev.n > SMALL_NODES) return 0;
+    most = std::max(most, h.dev.n);
+  }
+  return most;
+}
+
 std::vector<SweepItem> Batch::sweep_items(const nflow_tuning& t) const {
   if (storage != NFLOW_STORAGE_F32) return {};
   std::vector<nflow_input> in;
@@ -778,12 +780,12 @@ int Batch::autotune(int trial_steps, nflow_tuning* out) {
   nflow_tuning best = cand[0];
   for (const auto& t : cand)
     if (t.ms_per_step < best.ms_per_step) best = t;
-  // two steps per launch (where the batch allows it): the automatic choice
+  // several steps per launch (where the batch allows it): the automatic choice
   // and a few fixed chunk heights, each timed over pairs with the best shape
   nflow_tuning probe = best;
   probe.temporal = -1;
   std::vector<int> hs;
-  if (!sweep_items(probe).empty()) hs.push_back(-1);
+  if (small_nodes(probe) > 0 || !sweep_items(probe).empty()) hs.push_back(-1);
   for (int hh : {8, 16, 24, 32, 64}) {
     probe.temporal = hh;
     if (!sweep_items(probe).empty()) hs.push_back(hh);
