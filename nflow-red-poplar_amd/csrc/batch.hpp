@@ -150,6 +150,7 @@ class Batch {
   size_t device_bytes() const;
 
  private:
+  std::vector<nflow_input> plain_inputs() const;
   int ensure_scratch(size_t aos, size_t macro, size_t partials, size_t types);
   int build_graph(hipGraphExec_t* out, int parity, int steps);
 };

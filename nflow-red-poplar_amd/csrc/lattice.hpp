@@ -92,13 +92,6 @@ struct alignas(16) WorkItem {
   uint32_t pad;
 };
 
-// k_small: whole lattices of up to SMALL_NODES nodes in a workgroup's LDS.  One
-// compute unit's work per step meets the launch it saves near 2,000 nodes: us
-// per step of one step per launch / k_small, MRT, 512 nodes 3.8 / 1.2, 1000 4.0
-// / 1.75, 1100 4.0 / 2.3, 1728 4.1 / 3.1, 2028 4.1 / 3.8, 2048 in a row 3.65 /
-// 3.8.
-enum : int { SMALL_NT = 1024, SMALL_NODES = 1920 };
-
 // Kernel launchers (kernels.hip).
 // `steps` steps in one launch (k_small) of nlat FP32 cavities without solid
 // nodes, of at most `most` <= SMALL_NODES nodes each: reads buf[parity ^

@@ -350,7 +350,7 @@ int Batch::upload_tables() {
   if (!items.empty())
     NFLOW_HIP(hipMemcpy(d_items, items.data(), items.size() * sizeof(WorkItem), hipMemcpyHostToDevice));
   small = small_nodes(tuning);
-  const std::vector<SweepItem> sw = sweep_items(tuning);
+  const std::vector<SweepItem> sw = small > 0 ? std::vector<SweepItem>() : sweep_items(tuning);
   nsweep = 0;
   sweep_channel = false;
   sweep_runs = true;
@@ -713,24 +713,24 @@ int Batch::step2_height(const nflow_tuning* t) const {
   return best;
 }
 
-// Whole lattices in LDS, many steps per launch (k_small): where every lattice fits.
-uint32_t Batch::small_nodes(const nflow_tuning& t) const {
-  if (t.temporal >= 0 || storage != NFLOW_STORAGE_F32) return 0;
-  uint32_t most = 0;
-  for (const auto& h : lats) {
-    if (h.in.casetype != NFLOW_CAVITY || h.dev.mask || h.dev.n > SMALL_NODES) return 0;
-    most = std::max(most, h.dev.n);
-  }
-  return most;
-}
-
-std::vector<SweepItem> Batch::sweep_items(const nflow_tuning& t) const {
-  if (storage != NFLOW_STORAGE_F32) return {};
+// The lattices' inputs where kernels of several steps per launch take them: all
+// FP32 and without solid nodes; else none.
+std::vector<nflow_input> Batch::plain_inputs() const {
   std::vector<nflow_input> in;
+  if (storage != NFLOW_STORAGE_F32) return in;
   for (const auto& h : lats) {
     if (h.dev.mask) return {};
     in.push_back(h.in);
   }
+  return in;
+}
+
+uint32_t Batch::small_nodes(const nflow_tuning& t) const {
+  return (uint32_t)small_plan(plain_inputs(), cu_count, t.temporal);
+}
+
+std::vector<SweepItem> Batch::sweep_items(const nflow_tuning& t) const {
+  const std::vector<nflow_input> in = plain_inputs();
   return sweep_work(in, sweep_plan(in, cu_count, t.temporal));
 }
 

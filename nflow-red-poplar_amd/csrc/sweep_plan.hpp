@@ -1,5 +1,6 @@
 // sweep_plan.hpp -- which lattices take two steps per launch (k_sweep), in
-// which tiles and chunks of planes.  Host code without HIP.
+// which tiles and chunks of planes, and which many (k_small).  Host code
+// without HIP.
 #pragma once
 #include <vector>
 
@@ -39,5 +40,16 @@ std::vector<SweepShape> sweep_plan(const std::vector<nflow_input>& lats, int cu_
 
 // The work list of a plan.
 std::vector<SweepItem> sweep_work(const std::vector<nflow_input>& lats, const std::vector<SweepShape>& plan);
+
+// k_small: whole lattices of up to SMALL_NODES nodes in a workgroup's LDS.  One
+// compute unit's work per step meets the launch it saves near 2,000 nodes: us
+// per step of one step per launch / k_small, MRT, 512 nodes 3.8 / 1.2, 1000 4.0
+// / 1.75, 1100 4.0 / 2.3, 1728 4.1 / 3.1, 2028 4.1 / 3.8, 2048 in a row 3.65 /
+// 3.8.
+enum : int { SMALL_NT = 1024, SMALL_NODES = 1920 };
+
+// Many steps per launch for FP32 cavities without solid nodes: the nodes of the
+// largest where all are to run in k_small, else 0.
+int small_plan(const std::vector<nflow_input>& lats, int cu_count, int temporal);
 
 }  // namespace nflow

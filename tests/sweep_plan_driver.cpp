@@ -1,7 +1,8 @@
 // The plan of two-step launches (csrc/sweep_plan.cpp) for a batch given as
 // arguments (tests/test_sweep_plan_cpu.py): CUs, nflow_tuning.temporal, then
 // nx ny nz casetype per lattice.  Prints "tx tz h workgroups" per lattice (one
-// line "none" without a plan) after checking the work list: tiles within the
+// line "none" without a plan, "small" and the nodes of the largest where the
+// lattices run in k_small) after checking the work list: tiles within the
 // kernel's limits, each node in exactly one.
 #include <algorithm>
 #include <cstdio>
@@ -28,6 +29,10 @@ int main(int argc, char** argv) {
     i.nz = std::atoi(argv[a + 2]);
     i.casetype = std::atoi(argv[a + 3]);
     in.push_back(i);
+  }
+  if (const int n = small_plan(in, std::atoi(argv[1]), std::atoi(argv[2]))) {
+    std::printf("small %d\n", n);
+    return 0;
   }
   const auto plan = sweep_plan(in, std::atoi(argv[1]), std::atoi(argv[2]));
   if (plan.empty()) {

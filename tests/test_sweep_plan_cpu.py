@@ -1,4 +1,4 @@
-"""The choice of two steps per launch, its tiles and its chunk heights
+"""The choice of two or many steps per launch, its tiles and its chunk heights
 (csrc/sweep_plan.cpp), without a GPU: the driver checks every work list against
 the kernel's limits; here, which lattices get one."""
 import os
@@ -28,6 +28,8 @@ def plan(tmp_path_factory):
         r = subprocess.run([exe, str(cus), str(temporal)] + [str(v) for s in lats for v in s], capture_output=True,
                            text=True, timeout=60)
         assert r.returncode == 0, (lats, temporal, r.stderr)
+        if r.stdout.startswith("small"):
+            return int(r.stdout.split()[1])
         return None if r.stdout == "none\n" else [tuple(map(int, w.split())) for w in r.stdout.splitlines()]
 
     return run
@@ -107,3 +109,17 @@ def test_batches_take_two_steps_only_where_they_are_faster(plan):
     assert plan([(47, 47, 47, CH)] * 26) is None  # 79.8 and 88.8
     assert plan([(48, 48, 48, CAV)] * 16)  # 51.7 and 39.4
     assert plan([(77, 77, 77, CH)] * 6)  # 0.82 of one step's time
+
+
+def test_lattices_in_lds_only_where_they_are_faster(plan):
+    small = (10, 10, 10, CAV)
+    assert plan([small]) == 1000 and plan([small], temporal=0) is None
+    assert plan([(1920, 1, 1, CAV)]) == 1920 and plan([(1921, 1, 1, CAV)]) is None
+    assert plan([small, (12, 12, 12, CAV)]) == 1728
+    assert plan([small, (10, 10, 10, CH)]) is None and plan([small, (16, 16, 16, CAV)]) is None
+    # us per step of one step per launch / k_small
+    assert plan([(4, 4, 4, CAV)] * 1024) == 64  # 3.8 / 3.7
+    assert plan([(4, 4, 4, CAV)] * 4096) is None  # 9.4 / 14.7
+    assert plan([(3, 3, 3, CAV)] * 2048) is None  # 5.0 / 8.2
+    assert plan([(5, 5, 5, CAV)] * 4096) == 125  # 19.3 / 15.8
+    assert plan([(8, 8, 8, CAV)] * 4096) == 512  # 59 / 20
