@@ -141,15 +141,13 @@ class Batch {
   // 256 x 8 node tiles, resolving temporal = -1 by an estimate for those; 0:
   // none
   int step2_height(const nflow_tuning* t = nullptr) const;
-  // nodes of the largest lattice where all run in k_small under `t`, else 0
-  uint32_t small_nodes(const nflow_tuning& t) const;
-  // work list of two-step launches under `t`, empty for one step per launch
-  std::vector<SweepItem> sweep_items(const nflow_tuning& t) const;
   void destroy_graphs();
   long long total_nodes() const;
   size_t device_bytes() const;
 
  private:
+  // the inputs as sweep_plan and small_plan take them: all lattices' where they
+  // are FP32 and without solid nodes, else none
   std::vector<nflow_input> plain_inputs() const;
   int ensure_scratch(size_t aos, size_t macro, size_t partials, size_t types);
   int build_graph(hipGraphExec_t* out, int parity, int steps);

@@ -349,8 +349,10 @@ int Batch::upload_tables() {
     NFLOW_HIP(hipMemcpy(d_lats, devs.data(), devs.size() * sizeof(LatticeDev), hipMemcpyHostToDevice));
   if (!items.empty())
     NFLOW_HIP(hipMemcpy(d_items, items.data(), items.size() * sizeof(WorkItem), hipMemcpyHostToDevice));
-  small = small_nodes(tuning);
-  const std::vector<SweepItem> sw = small > 0 ? std::vector<SweepItem>() : sweep_items(tuning);
+  const std::vector<nflow_input> in = plain_inputs();
+  small = (uint32_t)small_plan(in, cu_count, tuning.temporal);
+  std::vector<SweepItem> sw;
+  if (small == 0) sw = sweep_work(in, sweep_plan(in, cu_count, tuning.temporal));
   nsweep = 0;
   sweep_channel = false;
   sweep_runs = true;
@@ -713,25 +715,15 @@ int Batch::step2_height(const nflow_tuning* t) const {
   return best;
 }
 
-// The lattices' inputs where kernels of several steps per launch take them: all
-// FP32 and without solid nodes; else none.
 std::vector<nflow_input> Batch::plain_inputs() const {
   std::vector<nflow_input> in;
   if (storage != NFLOW_STORAGE_F32) return in;
+  in.reserve(lats.size());
   for (const auto& h : lats) {
     if (h.dev.mask) return {};
     in.push_back(h.in);
   }
   return in;
-}
-
-uint32_t Batch::small_nodes(const nflow_tuning& t) const {
-  return (uint32_t)small_plan(plain_inputs(), cu_count, t.temporal);
-}
-
-std::vector<SweepItem> Batch::sweep_items(const nflow_tuning& t) const {
-  const std::vector<nflow_input> in = plain_inputs();
-  return sweep_work(in, sweep_plan(in, cu_count, t.temporal));
 }
 
 // Times every candidate launch shape on this batch's own lattices and keeps
@@ -782,14 +774,10 @@ int Batch::autotune(int trial_steps, nflow_tuning* out) {
     if (t.ms_per_step < best.ms_per_step) best = t;
   // several steps per launch (where the batch allows it): the automatic choice
   // and a few fixed chunk heights, each timed over pairs with the best shape
-  nflow_tuning probe = best;
-  probe.temporal = -1;
+  const std::vector<nflow_input> in = plain_inputs();
   std::vector<int> hs;
-  if (small_nodes(probe) > 0 || !sweep_items(probe).empty()) hs.push_back(-1);
-  for (int hh : {8, 16, 24, 32, 64}) {
-    probe.temporal = hh;
-    if (!sweep_items(probe).empty()) hs.push_back(hh);
-  }
+  for (int hh : {-1, 8, 16, 24, 32, 64})
+    if (small_plan(in, cu_count, hh) > 0 || !sweep_plan(in, cu_count, hh).empty()) hs.push_back(hh);
   if (!hs.empty()) {
     std::vector<nflow_tuning> tc;
     for (int hh : hs) {

@@ -92,6 +92,10 @@ static std::vector<std::pair<int, int>> sweep_tiles(const nflow_input& in) {
   return out;
 }
 
+static bool same_box(const nflow_input& a, const nflow_input& b) {
+  return a.nx == b.nx && a.ny == b.ny && a.nz == b.nz && a.casetype == b.casetype;
+}
+
 std::vector<SweepShape> sweep_plan(const std::vector<nflow_input>& lats, int cu_count, int temporal) {
   std::vector<SweepShape> none;
   // a chunk height is a choice for one lattice; batches of several choose
@@ -129,6 +133,10 @@ std::vector<SweepShape> sweep_plan(const std::vector<nflow_input>& lats, int cu_
     single += two_steps_us(in);
     pair += rounds * sweep_wg_us(in, shape[0], (double)shape[0].wgs / ((double)rounds * cu_count));
   } else {
+    for (const auto& in : lats) single += two_steps_us(in);
+    // a workgroup takes 2.97 + 1.28 x 2.81 us at least: many tiny lattices
+    // need no search
+    if (6.5 * lats.size() / cu_count >= single) return none;
     // every CU takes workgroups until none are left: the launch lasts as long
     // as their sum spread over the CUs, plus half of the longest at its end
     double best = 1e30;
@@ -137,16 +145,20 @@ std::vector<SweepShape> sweep_plan(const std::vector<nflow_input>& lats, int cu_
       double sum = 0.0, longest = 0.0;
       for (size_t i = 0; i < lats.size(); ++i) {
         const nflow_input& in = lats[i];
-        const int h = even_height(in.ny, std::min(cap, sweep_max_height(in)));
-        double least = 1e30;
-        for (const auto& tile : sweep_tiles(in)) {
-          const SweepShape s = sweep_shape(in, tile.first, tile.second, h);
-          if (s.wgs * s.at(1.0) < least) {
-            least = s.wgs * s.at(1.0);
-            c[i] = s;
+        if (i > 0 && same_box(in, lats[i - 1])) {
+          c[i] = c[i - 1];
+        } else {
+          const int h = even_height(in.ny, std::min(cap, sweep_max_height(in)));
+          double least = 1e30;
+          for (const auto& tile : sweep_tiles(in)) {
+            const SweepShape s = sweep_shape(in, tile.first, tile.second, h);
+            if (s.wgs * s.at(1.0) < least) {
+              least = s.wgs * s.at(1.0);
+              c[i] = s;
+            }
           }
         }
-        sum += least;
+        sum += c[i].wgs * c[i].at(1.0);
         longest = std::max(longest, c[i].at(1.0));
       }
       const double us = (sum / cu_count + 0.5 * longest) * SWEEP_ROUNDS;
@@ -161,7 +173,6 @@ std::vector<SweepShape> sweep_plan(const std::vector<nflow_input>& lats, int cu_
       const double us = sweep_wg_us(lats[i], shape[i], 1.0);
       sum += shape[i].wgs * us;
       longest = std::max(longest, us);
-      single += two_steps_us(lats[i]);
     }
     pair += sum / cu_count + 0.5 * longest;
   }
