@@ -71,11 +71,12 @@ inline void parallel_memcpy(void* dst, const void* src, size_t n) {
   run_threads(helpers_out(n), work, [&](int) { work(); });
 }
 
-// Pinned chunks and the events of the copies through them.
+// Pinned host memory: a block for one short copy, or chunks and the events of
+// the copies through them.
 struct Pinned {
-  static constexpr size_t CHUNK = 2u << 20, SLOTS = 8;
+  static constexpr size_t CHUNK = 2u << 20, SLOTS = 8, BLOCK = 1u << 20;
   char* buf = nullptr;
-  int device = -1;  // the events' device
+  int device = -1;  // the events' device; -1: a block, without events
   hipEvent_t ev[SLOTS] = {};
   Pinned() = default;
   Pinned(const Pinned&) = delete;
@@ -88,19 +89,22 @@ struct Pinned {
   bool open(int dev) {
     device = dev;
     bool ok = true;
-    for (auto& e : ev) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+    if (dev >= 0)
+      for (auto& e : ev) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
     void* p = nullptr;
-    ok = ok && hipHostMalloc(&p, SLOTS * CHUNK, hipHostMallocPortable) == hipSuccess;
+    ok = ok && hipHostMalloc(&p, dev >= 0 ? SLOTS * CHUNK : BLOCK, hipHostMallocPortable) == hipSuccess;
     if (!ok) (void)hipGetLastError();
     buf = ok ? static_cast<char*>(p) : nullptr;
     return ok;
   }
 };
 
-// The idle Pinned of the process, two at most, kept while any HostCopy lives
-// and given back with the last: a new solver's first read-back finds them
-// ready (allocating 16 MiB of pinned memory takes 1 to 2 ms).  Copies that
-// overlap each hold one of their own.
+// The process's pinned memory, at most 4 sets of chunks and 16 blocks (80 MiB),
+// kept while any HostCopy lives and given back with the last: a new solver's
+// first read-back finds it ready.  Copies that overlap each hold one of their
+// own; those that find none left are plain ones.  (Sets made for a third copy
+// at a time and freed after it: 8 threads that read 64^3 fields 1.9 ms at the
+// 90th percentile, and 1.15 with plain copies alone.)
 class PinnedPool {
  public:
   static std::shared_ptr<PinnedPool> get() {
@@ -111,19 +115,13 @@ class PinnedPool {
     if (!p) pool = p = std::make_shared<PinnedPool>();
     return p;
   }
-  std::unique_ptr<Pinned> take(int device) {
-    {
-      std::lock_guard<std::mutex> lk(mu_);
-      for (auto& p : idle_)
-        if (p && p->device == device) return std::move(p);
-    }
-    std::unique_ptr<Pinned> p(new (std::nothrow) Pinned);
-    if (p && !p->open(device)) p.reset();
-    return p;
-  }
+  // a set of chunks for `device`
+  std::unique_ptr<Pinned> take_chunks(int device) { return take(chunks_, device, true); }
+  // a block; grow: make one where none is idle
+  std::unique_ptr<Pinned> take_block(bool grow) { return take(blocks_, -1, grow); }
   void give(std::unique_ptr<Pinned> p) {
     std::lock_guard<std::mutex> lk(mu_);
-    for (auto& q : idle_)
+    for (auto& q : p->device < 0 ? blocks_.idle : chunks_.idle)
       if (!q) {
         q = std::move(p);
         return;
@@ -131,8 +129,36 @@ class PinnedPool {
   }
 
  private:
+  struct Kind {
+    std::unique_ptr<Pinned> idle[16];
+    int live, most;  // made and not freed; how many there may be
+  };
+  std::unique_ptr<Pinned> take(Kind& k, int device, bool grow) {
+    std::unique_ptr<Pinned> other;  // another device's, in the way
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      for (auto& p : k.idle)
+        if (p && p->device == device) return std::move(p);
+      if (!grow) return nullptr;
+      if (k.live == k.most) {
+        for (auto& p : k.idle)
+          if (p) other = std::move(p);
+        if (!other) return nullptr;
+        --k.live;
+      }
+      ++k.live;
+    }
+    other.reset();
+    std::unique_ptr<Pinned> p(new (std::nothrow) Pinned);
+    if (p && !p->open(device)) p.reset();
+    if (!p) {
+      std::lock_guard<std::mutex> lk(mu_);
+      --k.live;
+    }
+    return p;
+  }
   std::mutex mu_;
-  std::unique_ptr<Pinned> idle_[2];
+  Kind chunks_{{}, 0, 4}, blocks_{{}, 0, 16};
 };
 
 // One batch's copies: one host thread at a time, on the batch's stream and
@@ -146,7 +172,8 @@ class HostCopy {
   int to_host(hipStream_t st, const void* src, size_t n, void* const* dst, int parts) {
     const size_t total = n * parts;
     const int helpers = helpers_out(total);
-    const Lease lease(*this, helpers > 0 || total <= SMALL);
+    const Lease lease(*this, helpers > 0 ? CHUNKS : total > Pinned::BLOCK ? NONE : total > TINY || !first_ ? GROW : IDLE);
+    first_ = false;
     if (!lease) {  // plain copies
       for (int i = 0; i < parts; ++i)
         NFLOW_HIP(hipMemcpyAsync(dst[i], static_cast<const char*>(src) + i * n, n, hipMemcpyDeviceToHost, st));
@@ -236,7 +263,7 @@ class HostCopy {
   // reused on return (the last chunks may still be on their way).
   int to_device(hipStream_t st, void* dst, const void* src, size_t n) {
     const int most = helpers_in(n);
-    const Lease lease(*this, most > 0);
+    const Lease lease(*this, most > 0 ? CHUNKS : NONE);
     if (!lease) {
       NFLOW_HIP(hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, st));
       NFLOW_HIP(hipStreamSynchronize(st));
@@ -294,13 +321,21 @@ class HostCopy {
 
  private:
   static constexpr size_t CHUNK = Pinned::CHUNK, SLOTS = Pinned::SLOTS, PIECE = 256u << 10, PER = CHUNK / PIECE,
-                          SMALL = 1u << 20;
+                          TINY = 4u << 10;
   std::shared_ptr<PinnedPool> pool_ = PinnedPool::get();
+  // no copy to the host yet: a first one of up to TINY bytes that finds no idle
+  // block goes plain (the first diagnostics of a process 190 -> 75 us; making a
+  // block of 1 MiB takes some 70 us, a set of chunks 130)
+  bool first_ = true;
 
+  // what a copy takes from the pool: nothing, chunks, a block, a block only if one is idle
+  enum Want { NONE, CHUNKS, GROW, IDLE };
   // a Pinned of the pool for one copy (where wanted and to be had); every copy
   // through it has ended when it goes back
   struct Lease {
-    Lease(HostCopy& h, bool want) : pool(*h.pool_), p(want ? pool.take(h.device) : nullptr) {}
+    Lease(HostCopy& h, Want w)
+        : pool(*h.pool_),
+          p(w == NONE ? nullptr : w == CHUNKS ? pool.take_chunks(h.device) : pool.take_block(w == GROW)) {}
     ~Lease() {
       if (p) pool.give(std::move(p));
     }

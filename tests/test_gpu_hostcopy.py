@@ -2,7 +2,8 @@
 populations written and read back unchanged at sizes on either side of the
 plain, single and chunked paths (1 and 3 MiB out, 32 MiB in), of one chunk (2
 MiB) and of all eight (16 MiB, where chunks are used again), into views that start off any
-boundary; and from two host threads at once."""
+boundary; and from several host threads at once, more than the pool has pinned
+memory for among them."""
 import threading
 
 import numpy as np
@@ -56,3 +57,31 @@ def test_two_host_threads_at_once():
     for x in t:
         x.join()
     assert ok == {0: True, 1: True, 2: True}
+
+
+@pytest.mark.parametrize("count,n", [(18, (12, 11, 10)), (6, (50, 49, 48))])
+def test_more_copies_at_once_than_the_pool_holds(count, n):
+    """16 blocks and 4 sets of chunks: the others take plain copies."""
+    solvers = [nflow.Solver(nflow.defaults(**cfg(nx=n[0], ny=n[1], nz=n[2]), storage=nflow.F32)) for _ in range(count)]
+    given = [field((n[1] + 2, n[2] + 2, n[0] + 2, 19), k) for k in range(count)]
+    gate = threading.Barrier(count)
+    ok = [False] * count
+
+    def work(k):
+        gate.wait()
+        good = True
+        for _ in range(8):
+            solvers[k].write_arF(given[k])
+            good = good and np.array_equal(solvers[k].read_arF(), given[k])
+            mass = given[k].sum(dtype=np.float64)  # rho: 19 terms added in FP32
+            good = good and abs(solvers[k].diagnostics()[0] - mass) < 19 * 2.0 ** -24 * mass
+        ok[k] = good
+
+    t = [threading.Thread(target=work, args=(k,)) for k in range(count)]
+    for x in t:
+        x.start()
+    for x in t:
+        x.join()
+    for s in solvers:
+        s.close()
+    assert all(ok)
