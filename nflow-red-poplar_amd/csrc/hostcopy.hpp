@@ -259,14 +259,14 @@ class HostCopy {
     return 0;
   }
 
-  // n bytes from the host to dst on the device, in stream order; src may be
-  // reused on return (the last chunks may still be on their way).
+  // n bytes from the host to dst on the device, in stream order; src is free
+  // once the stream has been waited for.  (The chunks go back to the pool on
+  // return, so a copy through them has ended then.)
   int to_device(hipStream_t st, void* dst, const void* src, size_t n) {
     const int most = helpers_in(n);
     const Lease lease(*this, most > 0 ? CHUNKS : NONE);
     if (!lease) {
       NFLOW_HIP(hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, st));
-      NFLOW_HIP(hipStreamSynchronize(st));
       return 0;
     }
     char* const buf = lease->buf;

@@ -658,11 +658,10 @@ int Batch::import_one(int idx, const float* aos_host, long long step0) {
   int rc = ensure_scratch(padded_count(h.in), 0, 0, 0);
   if (rc) return rc;
   rc = host.to_device(stream, d_aos, aos_host, padded_count(h.in) * sizeof(float));
-  if (rc) return rc;
-  rc = init_lattice(idx, d_aos, step0);
-  if (rc) return rc;
-  NFLOW_HIP(hipStreamSynchronize(stream));
-  return 0;
+  if (!rc) rc = init_lattice(idx, d_aos, step0);
+  const hipError_t last = hipStreamSynchronize(stream);  // the caller's array may go
+  if (!rc) NFLOW_HIP(last);
+  return rc;
 }
 
 int Batch::node_types(int idx, int* type, int* dirstate) {
