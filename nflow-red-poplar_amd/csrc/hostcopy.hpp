@@ -32,7 +32,7 @@ namespace nflow {
 // cannot be had (f must do all the work that is left, whoever calls it).
 template <class F, class Main>
 void run_threads(int extra, F f, Main mine) {
-  constexpr int MOST = 8;
+  constexpr int MOST = 3;
   std::thread t[MOST];
   int n = 0;
   try {
@@ -53,11 +53,11 @@ inline int helpers_out(size_t bytes) {
 }
 
 // Helpers for a copy out of the caller's pages, which mostly are there: 67 MB
-// 2.6 -> 2.0 ms, but 9.5 MB 300 us as the runtime's own copy and 370 to 750
-// through the chunks.
+// 2.6 -> 1.95 ms, 323 MB 35 -> 8.2 (eight helpers: 1.98 and 8.3), but 9.5 MB 300
+// us as the runtime's own copy and 370 to 750 through the chunks.
 inline int helpers_in(size_t bytes) {
   const unsigned hw = std::thread::hardware_concurrency();
-  return bytes < (32u << 20) ? 0 : (int)std::min<size_t>(8, hw ? hw : 1);
+  return bytes < (32u << 20) ? 0 : (int)std::min<size_t>(3, hw ? hw : 1);
 }
 
 // memcpy by several threads (fresh destination pages are faulted in by all)
