@@ -16,10 +16,10 @@
 #include <atomic>
 #include <cstddef>
 #include <cstring>
+#include <exception>
 #include <memory>
 #include <mutex>
 #include <new>
-#include <system_error>
 #include <thread>
 #include <utility>
 
@@ -28,8 +28,9 @@
 
 namespace nflow {
 
-// Runs f() on `extra` more threads and on this one; fewer where threads
-// cannot be had (f must do all the work that is left, whoever calls it).
+// Runs f() on `extra` more threads (three at most) while this one runs
+// mine(their number); fewer where threads or their memory cannot be had (f must
+// do all the work that is left, whoever calls it).
 template <class F, class Main>
 void run_threads(int extra, F f, Main mine) {
   constexpr int MOST = 3;
@@ -37,7 +38,7 @@ void run_threads(int extra, F f, Main mine) {
   int n = 0;
   try {
     for (; n < std::min(extra, MOST); ++n) t[n] = std::thread(f);
-  } catch (const std::system_error&) {
+  } catch (const std::exception&) {  // system_error or bad_alloc
   }
   mine(n);
   for (int i = 0; i < n; ++i) t[i].join();
