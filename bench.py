@@ -545,9 +545,7 @@ def main():
     n = w["nx"] * w["ny"] * w["nz"]
     mlups = n * args.steps / wall / 1e6
     bpu = BYTES_PER_UPDATE[w["storage"]]
-    # every FP32 workload above is a cavity or channel that the library advances
-    # two steps per launch unless its tuning says otherwise
-    two = w["storage"] == 0 and b.get_tuning()["temporal"] != 0
+    two = h2 > 0
     if two:
         # the dominant kernel is k_sweep (two steps per launch, one read and one
         # write of the populations); its launch time from two runs of 2m + 1

@@ -228,12 +228,15 @@ int nflow_batch_get_tuning(nflow_batch* b, nflow_tuning* t);
 /* launch shape of a single-lattice solver (it is a batch of one; no
  * reference counterpart): the same fields and rules as for a batch */
 int nflow_set_tuning(nflow_solver* s, const nflow_tuning* t);
-/* chunk height that the batch's tuning names for two steps per launch: its
- * temporal where that is > 0, for -1 the estimate for tiles of 256 x 8 nodes,
- * 0 where that estimate finds one step per launch faster (and for batches of
- * several lattices, 16-bit storage and solid nodes).  With -1 a run may use
- * other tiles and heights than this, also where it is 0. */
+/* chunk height of the two-step launches that the batch's runs use under its
+ * tuning (of several lattices the tallest), 0 where they use none */
 int nflow_batch_step2_height(nflow_batch* b);
+/* launches of step kernels so far, those of captured graphs, of the autotuner
+ * and of read-backs that re-run a two-step launch among them: a run of n steps
+ * makes n of them with one step per launch, ceil(n / 2) with two (and one more
+ * for n even and the previous run read back), and one per 4,096 steps begun for
+ * small FP32 cavities, whose lattices stay in LDS meanwhile */
+long long nflow_batch_launches(nflow_batch* b);
 int nflow_batch_run(nflow_batch* b, int nsteps);
 int nflow_batch_synchronize(nflow_batch* b);
 int nflow_batch_read_arF(nflow_batch* b, int idx, float* dst);

@@ -85,7 +85,7 @@ class Batch {
   int replays = 0;  // of the short graphs
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   int last_steps = 0;
-  long long launches = 0;
+  long long launches = 0;  // of step kernels
   // the state of the last run was read back: the next run of an even number
   // of steps ends with single steps rather than a two-step launch
   bool read_back = false;
@@ -137,10 +137,8 @@ class Batch {
   int node_types(int idx, int* type, int* dirstate);
   int autotune(int trial_steps, nflow_tuning* out);
   int set_tuning(const nflow_tuning& t);
-  // y-chunk height that `t` (tuning by default) names for two-step launches of
-  // 256 x 8 node tiles, resolving temporal = -1 by an estimate for those; 0:
-  // none
-  int step2_height(const nflow_tuning* t = nullptr) const;
+  // tallest y chunk of the two-step launches of runs under `tuning`; 0: none
+  int step2_height() const;
   void destroy_graphs();
   long long total_nodes() const;
   size_t device_bytes() const;

@@ -677,41 +677,12 @@ int Batch::node_types(int idx, int* type, int* dirstate) {
   return 0;
 }
 
-int Batch::step2_height(const nflow_tuning* t) const {
-  const nflow_tuning& tu = t ? *t : tuning;
-  if (tu.temporal == 0 || storage != NFLOW_STORAGE_F32 || lats.size() != 1) return 0;
-  const HostLattice& h = lats[0];
-  if (h.in.casetype == NFLOW_PIPE || h.dev.mask) return 0;
-  if (tu.temporal > 0) return tu.temporal <= sweep_max_height(h.in) ? tu.temporal : 0;
-  // the height of least estimated time for tiles of 256 x 8 nodes, where that
-  // estimate beats 40 G node updates per second: one workgroup per CU, each
-  // sweeping its chunk's planes plus 0.86 at 12.18 + 2.70 w us per plane, w
-  // the share of the CUs busy in its round; times 0.84 + 0.16 fill for the
-  // idle lanes of partial x tiles and 1.21 for a channel's boundary records
-  constexpr int TX = 256, TZ = 8;
-  const int ntx = (h.in.nx + TX - 1) / TX;
-  const long cols = (long)ntx * ((h.in.nz + TZ - 1) / TZ);
-  const double fill = (double)h.in.nx / ((double)ntx * TX);
-  const double scale = (0.841 + 0.159 * fill) * (h.in.casetype == NFLOW_CHANNEL ? 1.213 : 1.0);
-  const double nodes = (double)h.in.nx * h.in.ny * h.in.nz;
-  double best_us = 2.0 * nodes / 40.0e3;  // two steps at 40 nodes per ns
-  int best = 0, prev = 0;
-  for (int cand : {8, 12, 16, 24, 32, 48, 64}) {
-    const int hh = std::min(cand, h.in.ny);
-    if (hh == prev || hh > sweep_max_height(h.in)) continue;
-    prev = hh;
-    const long nch = (h.in.ny + hh - 1) / hh;
-    const double planes = (double)h.in.ny / nch + 0.858;
-    double us = 0.0;
-    for (long left = cols * nch; left > 0; left -= cu_count)
-      us += planes * (12.184 + 2.696 * (double)std::min<long>(left, cu_count) / cu_count);
-    us *= scale;
-    if (us < best_us) {
-      best_us = us;
-      best = hh;
-    }
-  }
-  return best;
+int Batch::step2_height() const {
+  const std::vector<nflow_input> in = plain_inputs();
+  int h = 0;
+  if (small_plan(in, cu_count, tuning.temporal) == 0)
+    for (const SweepShape& s : sweep_plan(in, cu_count, tuning.temporal)) h = std::max(h, s.h);
+  return h;
 }
 
 std::vector<nflow_input> Batch::plain_inputs() const {
@@ -1159,6 +1130,8 @@ extern "C" int nflow_batch_step2_height(nflow_batch* b) {
   if (!b) return fail(NFLOW_EINVAL, "null batch");
   return b->b.step2_height();
 }
+
+extern "C" long long nflow_batch_launches(nflow_batch* b) { return b ? b->b.launches : -1; }
 
 extern "C" int nflow_batch_run(nflow_batch* b, int nsteps) {
   if (!b) return fail(NFLOW_EINVAL, "null batch");

@@ -106,6 +106,7 @@ SIGNATURES = {
     "nflow_batch_set_tuning": (_I, [_VP, ctypes.POINTER(Tuning)]),
     "nflow_batch_get_tuning": (_I, [_VP, ctypes.POINTER(Tuning)]),
     "nflow_batch_step2_height": (_I, [_VP]),
+    "nflow_batch_launches": (_LL, [_VP]),
     "nflow_set_tuning": (_I, [_VP, ctypes.POINTER(Tuning)]),
     "nflow_batch_run": (_I, [_VP, _I]),
     "nflow_batch_synchronize": (_I, [_VP]),
@@ -375,8 +376,12 @@ class Batch:
         return t.as_dict()
 
     def step2_height(self):
-        """y-chunk height its tuning names for two-step launches (see nflow_batch_step2_height)."""
+        """y-chunk height of the two-step launches its runs use (0: none)."""
         return _check(lib().nflow_batch_step2_height(self.h))
+
+    def launches(self):
+        """Step-kernel launches so far."""
+        return lib().nflow_batch_launches(self.h)
 
     def run(self, n):
         _check(lib().nflow_batch_run(self.h, n))

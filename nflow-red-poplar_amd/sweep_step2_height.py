@@ -5,7 +5,7 @@ fixed height, on this device.
 For each lattice (FP32, MRT-LES Cs 0.17; cavities tau 0.6, channels tau 0.56
 with a 0.05 inlet peak) it prints one JSON line: the rate in G node updates
 per second at temporal = 0 (one step per launch), -1 (the library's choice)
-and each fixed height, as [step2_height(), rate], from the library's HIP events
+and each fixed height, as [height used, rate], from the library's HIP events
 over 200 steps after 20.
 
     python nflow-red-poplar_amd/sweep_step2_height.py [--sizes 256x256x256,512x128x128c ...]

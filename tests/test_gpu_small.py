@@ -20,7 +20,8 @@ def inp(shape, vy=0.01, **kw):
                                 init_lid_velocity=1, **kw), storage=nflow.F32)
 
 
-def states(inputs, temporal, runs):
+def states(inputs, temporal, runs, launches=None):
+    """The states after each run; launches: of all runs (default: one a step)."""
     b = nflow.Batch(inputs)
     b.set_tuning(256, 0, 0, 10, temporal)
     b.initialize()
@@ -28,6 +29,7 @@ def states(inputs, temporal, runs):
     for n in runs:
         b.run(n)
         out += [(b.read_arF(i), b.diagnostics(i)) for i in range(len(inputs))]
+    assert b.launches() == (sum(runs) if launches is None else launches)
     b.close()
     return out
 
@@ -43,19 +45,20 @@ def same(a, b):
 def test_lattices_in_lds_equal_one_step_per_launch(shape, les):
     c = [inp(shape, enable_mrt=les, enable_les=les, smagorinsky=0.17 * les)]
     runs = [1, 2, 9, 12]
-    same(states(c, -1, runs), states(c, 0, runs))
+    fits = shape[0] * shape[1] * shape[2] <= 1920
+    same(states(c, -1, runs, launches=len(runs) if fits else None), states(c, 0, runs))
 
 
 def test_runs_longer_than_one_launch():
     # no lid velocity along y: the lid's (5 - 2)(6 - 2) nodes would take mass
     # out at every step, until none is left
     c = [inp((5, 4, 6), vy=0.0)]
-    same(states(c, -1, [4097, 8192]), states(c, 0, [4097, 8192]))
+    same(states(c, -1, [4097, 8192], launches=4), states(c, 0, [4097, 8192]))
 
 
 def test_a_batch_of_small_lattices_and_one_with_a_larger():
-    small = [inp(s, enable_mrt=i % 2) for i, s in enumerate(SHAPES)]
-    same(states(small, -1, [7, 10]), states(small, 0, [7, 10]))
+    small = [inp(s, enable_mrt=i % 2) for i, s in enumerate(SHAPES) if s != (17, 113, 1)]
+    same(states(small, -1, [7, 10], launches=2), states(small, 0, [7, 10]))
     mixed = small + [inp((16, 16, 16))]
     same(states(mixed, -1, [7, 10]), states(mixed, 0, [7, 10]))
 
@@ -79,4 +82,7 @@ def test_the_autotuner_times_and_keeps_it(count):
     """10^3 runs at 1.75 us per step in LDS and 3.3 with one step per launch."""
     b = nflow.Batch([inp((10, 10, 10))] * count)
     assert b.autotune(steps_per_trial=20)["temporal"] == -1
+    before = b.launches()
+    b.run(100)
+    assert b.launches() - before == 1
     b.close()

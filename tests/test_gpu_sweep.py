@@ -34,7 +34,7 @@ CASES = [
 ]
 
 
-def run(inputs, temporal, steps_list):
+def run(inputs, temporal, steps_list, launches):
     b = nflow.Batch(inputs)
     b.set_tuning(256, 0, 0, 0, temporal)
     b.initialize()
@@ -42,6 +42,7 @@ def run(inputs, temporal, steps_list):
     for n in steps_list:
         b.run(n)
         out += [(b.read_arF(i), b.diagnostics(i)[0]) for i in range(len(inputs))]
+    assert b.launches() == launches
     b.close()
     return out
 
@@ -55,9 +56,9 @@ def same(a, b):
 @pytest.mark.parametrize("k", range(len(CASES)))
 def test_row_tiles_equal_one_step_per_launch(k):
     inp = [nflow.defaults(**CASES[k], storage=nflow.F32)]
-    ref = run(inp, 0, [6, 5])
+    ref = run(inp, 0, [6, 5], 11)
     for h in (1, 2, 5, 200):
-        same(run(inp, h, [6, 5]), ref)
+        same(run(inp, h, [6, 5], 8), ref)  # 3 pairs, the last re-run as 2 steps, 2 pairs and 1 step
 
 
 @pytest.mark.parametrize("channels", [False, True])
@@ -68,4 +69,5 @@ def test_batches_of_several_lattices_equal_one_step_per_launch(channels):
               nflow.defaults(**cfg(nx=128, ny=96, nz=96, tau=0.53, **LES))]
     if channels:
         inputs.append(nflow.defaults(**channel(nx=300, ny=60, nz=64)))
-    same(run(inputs, -1, [8, 4, 7]), run(inputs, 0, [8, 4, 7]))
+    # 4 pairs, the last re-run as 2 steps; 1 pair and 2 steps; 3 pairs and 1 step
+    same(run(inputs, -1, [8, 4, 7], 13), run(inputs, 0, [8, 4, 7], 19))

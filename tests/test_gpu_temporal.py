@@ -1,4 +1,4 @@
-"""Two time steps per launch (nflow_tuning.temporal, k_step2; FP32 cavity and
+"""Two time steps per launch (nflow_tuning.temporal, k_sweep; FP32 cavity and
 channel lattices) against one step per launch: the same state bit for bit,
 for both collision models, partial tiles and y chunks, several x tiles, the
 channel's inlet and outlet in one or two tiles, tiny boxes, the benchmark
@@ -79,20 +79,22 @@ def test_two_steps_per_launch_at_256_cubed():
 
 
 def test_two_steps_per_launch_on_the_512x128x128_channel():
-    """The channel of the precision runs at its automatic chunk height (16):
-    two x tiles, inlet and outlet in different tiles, 8 y chunks."""
+    """The channel of the precision runs at its automatic tiles and chunk
+    height: inlet and outlet in different tiles, several y chunks."""
     c = cfg(nx=512, ny=128, nz=128, casetype=nflow.CHANNEL, enable_les=1, smagorinsky=0.17, tau=0.56,
             inlet_peak=0.05, perturb=0.01, seed=11)
     out = []
     for h in (0, -1):
         b = nflow.Batch([nflow.defaults(**c, storage=nflow.F32)])
         b.set_tuning(512, 0, 0, 0, h)
-        assert b.step2_height() == (0 if h == 0 else 16)
+        assert (b.step2_height() > 0) == (h != 0)
         b.initialize()
         got = []
         for n in (9, 6):
             b.run(n)
             got.append((b.read_macro(0), b.diagnostics(0)))
+        # 4 pairs and 1 step, then (the first state was read back) 2 pairs and 2
+        assert b.launches() == (15 if h == 0 else 9)
         b.close()
         out.append(got)
     for (m, d), (m2, d2) in zip(*out):
@@ -128,40 +130,35 @@ def test_temporal_is_ignored_where_it_does_not_apply():
         assert np.array_equal(x, y)
 
 
-def test_automatic_chunk_height():
-    """temporal = -1 (the default): the chunk height (8-64 planes) of the least
-    estimated launch time, two steps per launch only where the estimate beats
-    40 G node updates per second (256 CUs).  Each case's height is the fastest
-    measured among 8, 12, 16, 24, 32, 48 and 64, and each case left at one
-    step per launch measured no faster with two (within 1%; 128^3 7.6%)."""
-    def height(nx, ny, nz, storage=nflow.F32, casetype=nflow.CAVITY, temporal=-1):
+TWO, ONE = True, False
+
+
+@pytest.mark.parametrize("nx,ny,nz,casetype,two", [
+    (256, 256, 256, nflow.CAVITY, TWO), (256, 64, 256, nflow.CAVITY, TWO), (192, 192, 192, nflow.CAVITY, TWO),
+    (200, 300, 100, nflow.CAVITY, TWO), (288, 288, 288, nflow.CAVITY, TWO), (128, 128, 128, nflow.CAVITY, TWO),
+    (96, 96, 96, nflow.CAVITY, TWO), (48, 48, 48, nflow.CAVITY, ONE), (170, 4, 248, nflow.CAVITY, ONE),
+    (1024, 100, 1024, nflow.CAVITY, TWO),  # a plane has as many tiles as the chip has CUs
+    (512, 128, 128, nflow.CHANNEL, TWO), (320, 128, 128, nflow.CHANNEL, TWO), (274, 28, 24, nflow.CHANNEL, ONE),
+    (200, 60, 60, nflow.PIPE, ONE)])
+def test_automatic_choice(nx, ny, nz, casetype, two):
+    """temporal = -1 (the default): step2_height() is what a run does.  The
+    choice itself is checked without a GPU (tests/test_sweep_plan_cpu.py)."""
+    def batch(temporal=-1, storage=nflow.F32):
         b = nflow.Batch([nflow.defaults(**cfg(nx=nx, ny=ny, nz=nz, casetype=casetype), storage=storage)])
         b.set_tuning(512, 0, 0, 0, temporal)
-        h = b.step2_height()
+        b.initialize()
+        b.run(5)
+        out = b.step2_height(), b.launches()
         b.close()
-        return h
+        return out
+
     assert nflow.device_info()[1] == 256
-    assert height(256, 256, 256) == 32  # 32 tiles x 8 chunks
-    assert height(256, 128, 256) == 16
-    assert height(512, 256, 512) == 64  # 128 tiles x 4 chunks
-    assert height(256, 64, 256) == 8
-    assert height(256, 96, 256) == 12
-    assert height(192, 192, 192) == 24  # partial x tiles
-    assert height(384, 384, 384) == 48
-    assert height(200, 300, 100) == 16
-    assert height(128, 128, 128) == 0  # half the lanes idle
-    assert height(160, 160, 160) == 0
-    assert height(288, 288, 288) == 0  # second x tile an eighth full
-    assert height(512, 64, 64) == 0  # too few tiles for the CUs
-    assert height(48, 48, 48) == 0
-    assert height(256, 256, 256, storage=nflow.F16) == 0
-    assert height(512, 128, 128, casetype=nflow.CHANNEL) == 16  # 32 tiles x 8 chunks
-    assert height(768, 128, 128, casetype=nflow.CHANNEL) == 8
-    assert height(256, 128, 128, casetype=nflow.CHANNEL) == 8
-    assert height(320, 128, 128, casetype=nflow.CHANNEL) == 0
-    assert height(512, 128, 128, casetype=nflow.PIPE) == 0
-    assert height(256, 256, 256, temporal=24) == 24
-    assert height(256, 256, 256, temporal=0) == 0
+    h, launches = batch()
+    assert (h > 0) == two and h <= ny
+    assert launches == (3 if two else 5)
+    assert batch(temporal=0) == (0, 5)
+    assert batch(temporal=3) == ((0, 5) if casetype == nflow.PIPE else (3, 3))
+    assert batch(storage=nflow.F16) == (0, 5)
 
 
 @pytest.mark.parametrize("k", [0, 7])
