@@ -53,10 +53,10 @@ static constexpr double SWEEP_ROUNDS = 1.06;
 // lattices: chunks of few planes and CUs without work, where the estimate above
 // is up to 7 us short for channels.  For that question alone: us of a workgroup
 // of shape s when w of the CUs are busy, and us of two single steps.  Fitted,
-// with 4 us for the launch, to 900 cavities and channels of 30,000 to 2,000,000
-// nodes near the line (1.6 and 1.9 us rms, two single steps 5%).  On 400 others
-// the answer costs 0.6% against the faster of the two and 8 are more than 2%
-// slower; by the estimate above 3.5%, and 87 were slower, by up to 40%, channels
+// with 4 us for the launch, to 1,800 cavities and channels of 30,000 to 2,000,000
+// nodes near the line (1.6 and 1.9 us rms, two single steps 5%).  On 800 others
+// the answer costs 0.3% against the faster of the two, and 7 are more than 2%
+// slower; by the estimate above 2.7%, and 142 were slower, by up to 40%, channels
 // of some 100,000 nodes above all (274 x 28 x 24: 11.2 us a step, and 8.1 with
 // one step per launch).
 static double sweep_wg_us(const nflow_input& in, const SweepShape& s, double w) {
@@ -66,7 +66,8 @@ static double sweep_wg_us(const nflow_input& in, const SweepShape& s, double w) 
   const double planes = (double)in.ny / ((in.ny - 1) / s.h + 1) + 0.28;
   const double plane = ch ? 4.84 + 0.39 * halo + 2.93 * w * fill - (s.tx < in.nx ? 0.18 : 0.0)
                           : 2.81 + 1.29 * halo + 3.16 * w * fill + (s.tx < in.nx ? 0.21 : 0.0);
-  return (ch ? 4.95 + 4.36 * halo : 2.97 + 4.59 * halo) + planes * plane;
+  const double start = halo == 0.0 ? (ch ? 2.95 : 1.77) : ch ? 4.95 + 4.36 * halo : 2.97 + 4.59 * halo;
+  return start + planes * plane;
 }
 static double two_steps_us(const nflow_input& in) {
   const bool ch = in.casetype == NFLOW_CHANNEL;
@@ -131,12 +132,19 @@ std::vector<SweepShape> sweep_plan(const std::vector<nflow_input>& lats, int cu_
     }
     const long rounds = (shape[0].wgs - 1) / cu_count + 1;
     single += two_steps_us(in);
+    // cavities in narrow rows, of which a launch holds every node at once (three
+    // or, in rows on 128-byte lines, four workgroups of 256 a CU), take less
+    // (64^3 7.0 us a step, 7.8 in pairs; 61 x 15 x 213 6.9 and 8.1)
+    const bool lines = in.nx % 32 == 0;
+    if (in.casetype == NFLOW_CAVITY && in.nx <= 192 &&
+        (long long)in.nx * in.ny * in.nz <= (lines ? 1024ll : 768ll) * cu_count)
+      single *= lines ? 0.83 : 0.9;
     pair += rounds * sweep_wg_us(in, shape[0], (double)shape[0].wgs / ((double)rounds * cu_count));
   } else {
     for (const auto& in : lats) single += two_steps_us(in);
-    // a workgroup takes 2.97 + 1.28 x 2.81 us at least: many tiny lattices
+    // a workgroup takes 1.77 + 1.28 x 2.81 us at least: many tiny lattices
     // need no search
-    if (6.5 * lats.size() / cu_count >= single) return none;
+    if (5.3 * lats.size() / cu_count >= single) return none;
     // every CU takes workgroups until none are left: the launch lasts as long
     // as their sum spread over the CUs, plus half of the longest at its end
     double best = 1e30;

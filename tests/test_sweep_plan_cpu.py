@@ -92,7 +92,9 @@ MEASURED = [
     ((274, 28, 24, CH), 8.1, 11.2), ((322, 47, 19, CH), 10.7, 14.9), ((142, 12, 110, CH), 7.8, 10.6),
     ((56, 52, 62, CH), 7.7, 9.7), ((30, 36, 245, CH), 11.5, 13.5), ((211, 5, 181, CH), 7.4, 10.4),
     ((170, 4, 248, CAV), 7.4, 8.6), ((306, 13, 44, CAV), 8.0, 9.6), ((59, 13, 217, CAV), 6.6, 7.9),
-    ((194, 27, 32, CAV), 6.4, 8.3),
+    ((194, 27, 32, CAV), 6.4, 8.3), ((64, 64, 64, CAV), 7.0, 7.8), ((128, 64, 32, CAV), 7.0, 7.8),
+    ((61, 15, 213, CAV), 6.9, 8.1), ((64, 64, 64, CH), 8.8, 9.8), ((72, 72, 72, CAV), 12.3, 10.1),
+    ((60, 60, 60, CAV), 8.9, 7.9), ((76, 76, 76, CH), 15.6, 14.0),
     ((96, 96, 96, CAV), 25.6, 16.6), ((101, 67, 83, CAV), 17.9, 13.6), ((128, 128, 128, CAV), 53.5, 33.8),
     ((66, 62, 233, CH), 30.1, 22.7), ((44, 98, 246, CH), 34.2, 24.9), ((512, 128, 128, CH), 215.0, 125.4),
     ((30, 150, 104, CAV), 16.6, 12.4), ((179, 32, 154, CAV), 26.4, 18.1), ((28, 323, 96, CH), 27.8, 17.1),
