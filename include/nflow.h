@@ -213,9 +213,11 @@ typedef struct nflow_tuning {
    * then it ends with two single steps.  H > 0: that chunk height (batches of
    * one lattice; others take one step per launch); -1 (the default): tiles
    * and heights chosen by the library from an estimate of the launch time, on
-   * where that beats one step per launch (from about 56^3 nodes up; batches
-   * of several lattices by the sum of theirs); 0: one step per launch.  The
-   * autotuner times it. */
+   * where that beats one step per launch (cavities from about 60^3 nodes up,
+   * channels from about 72^3; batches of several lattices by the sum of
+   * theirs), and, for FP32 cavities of at most 1,920 nodes without solid ones,
+   * up to 4,096 steps per launch with each lattice in LDS; 0: one step per
+   * launch.  The autotuner times it. */
   int temporal;
   double ms_per_step; /* filled by the autotuner */
 } nflow_tuning;

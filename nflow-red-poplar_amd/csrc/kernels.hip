@@ -720,7 +720,7 @@ __global__ void __launch_bounds__(BS) NFLOW_STEP_ATTR k_step(const LatticeDev* _
 // Collision counters of the stochastic rounding: ctr[0] += steps for every
 // lattice.  Step launches carry their distance from ctr[0] as an argument, so
 // this runs once per graph replay, whose arguments are fixed, and not after
-// every step: at 48^3 FP16 a second 3.6 us launch per step (7.25 -> 3.7 us).
+// every step: 48^3 FP16 7.25 -> 5.8 us per step.
 #if NFLOW_STORAGE_SET != 2  // the FP32 object carries it
 __global__ void __launch_bounds__(256) k_advance(const LatticeDev* __restrict__ lats, int nlat, uint32_t steps) {
   const int i = blockIdx.x * 256 + threadIdx.x;
