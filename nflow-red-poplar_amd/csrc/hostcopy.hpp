@@ -143,7 +143,7 @@ class PinnedPool {
       if (!grow) return nullptr;
       if (k.live == k.most) {
         for (auto& p : k.idle)
-          if (p) other = std::move(p);
+          if (p && !other) other = std::move(p);
         if (!other) return nullptr;
         --k.live;
       }
